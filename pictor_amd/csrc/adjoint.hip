@@ -117,7 +117,13 @@ __global__ __launch_bounds__(256) void k_eng_push(AdjP ap, const typename V4<R>:
     int ei = di, ej = dj;   // cell of the second half-segment
     if constexpr (std::is_same<R, float>::value) {
         // the split form deposits as the production kernel: FP64 to the stored position
-        pushdev::zigzag2d_split(sp2(ap.qs, s), in.ox[p], in.oy[p], kZMid, ox, oy, q.x1[2], di, dj, a, b);
+        const pushdev::Zigzag zz(sp2(ap.qs, s), in.ox[p], in.oy[p], ox, oy, q.x1[2], di, dj);
+        for (int h = 0; h < 2; h++) {
+            unsigned long long m[8];
+            zz.jx(h, m); zz.jy(h, m + 2); zz.jz(h, m + 4);
+#pragma unroll
+            for (int k = 0; k < 8; k++) (h ? b : a)[k] = (double)(long long)m[k];
+        }
     } else {
         seg_values<R>(q.F1, q.W1, a);
         seg_values<R>(q.F2, q.W2, b);

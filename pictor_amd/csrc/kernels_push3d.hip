@@ -6,6 +6,12 @@
 // (i + a, j + b, k + c), nn = 1 + a + 2b + 4c), the 12-value zigzag deposit of
 // movdep.F90:187-234 into an LDS current window, the exchange of
 // loadprtlout.F90:22-97 with its z rules, and 27 arrival bins per tile.
+//
+// The loop is that of the 2-D kernels (one prefetched particle, its bin kept between
+// iterations, one LDS add for both halves of a move inside a cell).  The split form's deposit
+// makes one component's counts at a time: 75 instead of 91 VGPRs and 51 KB of LDS let three
+// workgroups share a CU instead of two.  128^3, 33.5M particles: push 684 -> 622 us (18.5 ps
+// per particle; VALU 74 %, LDS 72 % of the cycles); 48 x 40 x 32 in FP64 (tile 4): 60 -> 53 us.
 #include "pictor_common.h"
 #include "push_common.h"
 
@@ -40,8 +46,10 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
     const int mx = g.mx;
     const long long mxy = (long long)g.mx * g.my;
 
+    int bcnt = 0;
     if (tid < 27) {
         const int b = tile * tp.NB + tid;
+        bcnt = bins.cnt_in[b];
         sSrc[tid] = bins.base[b];
         const int ddx = tid % 3 - 1, ddy = (tid / 3) % 3 - 1, ddz = tid / 9 - 1;
         const int dt = (wrap_tile(tz + ddz, tp.ntz) * tp.nty + wrap_tile(ty + ddy, tp.nty)) * tp.ntx +
@@ -52,11 +60,7 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
         sDstCap[tid] = bins.cap[db];
         sCnt[tid] = 0;
     }
-    if (tid == 0) {
-        int acc = 0;
-        for (int b = 0; b < 27; b++) { sStart[b] = acc; acc += bins.cnt_in[tile * tp.NB + b]; }
-        sStart[27] = acc;
-    }
+    if (tid < 64) bin_starts(bcnt, 27, sStart);
     const double bx0 = ph.bext[0], by0 = ph.bext[1], bz0 = ph.bext[2];
     for (int e = tid; e < WN3; e += BS) {
         const int ii = e % WN, jj = (e / WN) % WN, kk = e / (WN * WN);
@@ -74,19 +78,37 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
 
     const double c = ph.c, sqc = ph.sqc, cinv = ph.cinv, qi = ph.qi;
     const int total = sStart[27];
+    // position k lies in bin `bin` while k < binEnd, at slot k + binOff; a thread's k only grows
+    int bin = 0, binEnd = sStart[1];
+    long long binOff = sSrc[0];
+    auto load = [&](int k, RecF64 &r) {
+        if (k >= binEnd) {
+            bin = bin_of<27>(k, sStart, 27);
+            binEnd = sStart[bin + 1];
+            binOff = sSrc[bin] - sStart[bin];
+        }
+        const long long src = binOff + k;
+        r.x = A.x[src]; r.y = A.y[src]; r.z = A.z[src];
+        r.u = A.u[src]; r.v = A.v[src]; r.w = A.w[src];
+        r.q = A.q[src]; r.flv = A.flv[src];
+        if (TAG) r.tag = A.tag[src];
+    };
+    RecF64 cur;
+    if (tid < total) load(tid, cur);
+    settle(cur.x, cur.y, cur.z, cur.u, cur.v, cur.w, cur.q, cur.flv);
     for (int base = 0; base < total; base += BS) {
         const int k = base + tid;
         const bool active = k < total;
-        double x0 = 0, y0 = 0, z0 = 0, un = 0, vn = 0, wn = 0, q = 0, xn = 0, yn = 0, zn = 0;
+        RecF64 nxt;
+        load(min(k + BS, total - 1), nxt);   // prefetch the next particle of this thread
+        double x0 = 0, y0 = 0, z0 = 0, un = 0, vn = 0, wn = 0, q = 0;
+        double xn = 0, yn = 0, zn = 0;
         int flv = 0, d = -1, tg = 0;
         if (active) {
-            const int b = bin_of<27>(k, sStart, 27);
-            const long long src = sSrc[b] + (k - sStart[b]);
-            x0 = A.x[src]; y0 = A.y[src]; z0 = A.z[src];
-            un = A.u[src]; vn = A.v[src]; wn = A.w[src];
-            q = A.q[src]; flv = A.flv[src];
-            if (TAG) tg = A.tag[src];
-            xn = x0; yn = y0; zn = z0;
+            x0 = cur.x; y0 = cur.y; z0 = cur.z;
+            un = cur.u; vn = cur.v; wn = cur.w;
+            q = cur.q; flv = cur.flv;
+            if (TAG) tg = cur.tag;
             const int ip0 = (int)x0, jp0 = (int)y0, kp0 = (int)z0;
             // node-window coordinates of the cell (origin i0-1)
             const int gi = ip0 - (i0 - 1), gj = jp0 - (j0 - 1), gk = kp0 - (k0 - 1);
@@ -138,30 +160,41 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
                 const double yr = dmin((double)(min(jp0, jp) + 1), dmax((double)max(jp0, jp), 0.5 * (y0 + yn)));
                 const double zr = dmin((double)(min(kp0, kp) + 1), dmax((double)max(kp0, kp), 0.5 * (z0 + zn)));
                 const double qthis = q * qi;
+                const double Fx[2] = {qthis * (xr - x0), qthis * (xn - xr)};
+                const double Fy[2] = {qthis * (yr - y0), qthis * (yn - yr)};
+                const double Fz[2] = {qthis * (zr - z0), qthis * (zn - zr)};
+                const double Wx[2] = {0.5 * (x0 + xr) - ip0, 0.5 * (xn + xr) - ip};
+                const double Wy[2] = {0.5 * (y0 + yr) - jp0, 0.5 * (yn + yr) - jp};
+                const double Wz[2] = {0.5 * (z0 + zr) - kp0, 0.5 * (zn + zr) - kp};
+                // a particle that stays in its cell deposits both halves on the same nodes: one
+                // LDS add for their sum
+                const bool cross = ip != ip0 || jp != jp0 || kp != kp0;
+                constexpr int sy = WJ, sz = WJ * WJ;
+                const int ea = ((kp0 - (k0 - 2)) * WJ + (jp0 - (j0 - 2))) * WJ + (ip0 - (i0 - 2));
+                const int eb = ((kp - (k0 - 2)) * WJ + (jp - (j0 - 2))) * WJ + (ip - (i0 - 2));
+                // F (1 - P, P) x (1 - Q, Q) on the nodes 0, sp, sq, sp + sq of a component
+                auto deposit = [&](double *w, const double *F, const double *P, const double *Q, int sp_, int sq_) {
+                    double v[2][4];
 #pragma unroll
-                for (int seg = 0; seg < 2; seg++) {
-                    const double xa = seg ? xn : x0, ya = seg ? yn : y0, za = seg ? zn : z0;
-                    const int ia = seg ? ip : ip0, ja = seg ? jp : jp0, ka = seg ? kp : kp0;
-                    const double Fx = seg ? qthis * (xn - xr) : qthis * (xr - x0);
-                    const double Fy = seg ? qthis * (yn - yr) : qthis * (yr - y0);
-                    const double Fz = seg ? qthis * (zn - zr) : qthis * (zr - z0);
-                    const double Wx = 0.5 * (xa + xr) - ia, Wy = 0.5 * (ya + yr) - ja, Wz = 0.5 * (za + zr) - ka;
-                    const int e = ((ka - (k0 - 2)) * WJ + (ja - (j0 - 2))) * WJ + (ia - (i0 - 2));
-                    constexpr int sy = WJ, sz = WJ * WJ;
-                    // Jx(i, j..j+1, k..k+1), Jy(i..i+1, j, k..k+1), Jz(i..i+1, j..j+1, k)
-                    atomicAdd(&sJ[0][e], (Fx * (1.0 - Wy)) * (1.0 - Wz));
-                    atomicAdd(&sJ[0][e + sy], (Fx * Wy) * (1.0 - Wz));
-                    atomicAdd(&sJ[0][e + sz], (Fx * (1.0 - Wy)) * Wz);
-                    atomicAdd(&sJ[0][e + sy + sz], (Fx * Wy) * Wz);
-                    atomicAdd(&sJ[1][e], (Fy * (1.0 - Wx)) * (1.0 - Wz));
-                    atomicAdd(&sJ[1][e + 1], (Fy * Wx) * (1.0 - Wz));
-                    atomicAdd(&sJ[1][e + sz], (Fy * (1.0 - Wx)) * Wz);
-                    atomicAdd(&sJ[1][e + 1 + sz], (Fy * Wx) * Wz);
-                    atomicAdd(&sJ[2][e], (Fz * (1.0 - Wx)) * (1.0 - Wy));
-                    atomicAdd(&sJ[2][e + 1], (Fz * Wx) * (1.0 - Wy));
-                    atomicAdd(&sJ[2][e + sy], (Fz * (1.0 - Wx)) * Wy);
-                    atomicAdd(&sJ[2][e + 1 + sy], (Fz * Wx) * Wy);
-                }
+                    for (int h = 0; h < 2; h++) {
+                        const double l = F[h] * (1.0 - P[h]), u = F[h] * P[h];
+                        v[h][0] = l * (1.0 - Q[h]); v[h][1] = u * (1.0 - Q[h]); v[h][2] = l * Q[h]; v[h][3] = u * Q[h];
+                    }
+                    if (!cross) {
+#pragma unroll
+                        for (int m = 0; m < 4; m++) v[0][m] = v[0][m] + v[1][m];
+                    }
+                    atomicAdd(w + ea, v[0][0]); atomicAdd(w + ea + sp_, v[0][1]);
+                    atomicAdd(w + ea + sq_, v[0][2]); atomicAdd(w + ea + sp_ + sq_, v[0][3]);
+                    if (cross) {
+                        atomicAdd(w + eb, v[1][0]); atomicAdd(w + eb + sp_, v[1][1]);
+                        atomicAdd(w + eb + sq_, v[1][2]); atomicAdd(w + eb + sp_ + sq_, v[1][3]);
+                    }
+                };
+                // Jx(i, j..j+1, k..k+1), Jy(i..i+1, j, k..k+1), Jz(i..i+1, j..j+1, k)
+                deposit(sJ[0], Fx, Wy, Wz, sy, sz);
+                deposit(sJ[1], Fy, Wx, Wz, 1, sz);
+                deposit(sJ[2], Fz, Wx, Wy, 1, sy);
                 // EnforceBC_PostMovDep (bc.F90:238-287)
                 bool keep = true;
                 if (BC) keep = particle_faces<double>(ph, g, xn, yn, zn, un, vn);
@@ -227,7 +260,8 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
                 }
             }
         }
-        const int slot = reserve_slot(d, sCnt);
+        const int slot = reserve_slot(d, 13, sCnt);
+        settle(nxt.x, nxt.y, nxt.z, nxt.u, nxt.v, nxt.w, nxt.q, nxt.flv);
         if (active && d >= 0) {
             if (slot < sDstCap[d]) {
                 const long long o = sDstBase[d] + slot;
@@ -247,6 +281,7 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
                 }
             }
         }
+        cur = nxt;
     }
     __syncthreads();
     for (int e = tid; e < WJ3; e += BS) {
@@ -264,10 +299,10 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
 // [i0, i0+T], current window [i0-1, i0+T+1].
 // ---------------------------------------------------------------------------
 struct SplitRec3 {
-    int cell, s;
+    int cell;
     float ox, oy, oz, u, v, w;
-    int id;     // the caller's tag (TAG only)
-    float wq;   // charge weight (WQ only)
+    int id;     // tag (TAG)
+    float wq;   // charge weight (WQ)
 };
 
 template <int T, int BS, bool BC, bool TAG = false, bool WQ = false>
@@ -282,6 +317,7 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
     constexpr int WN = T + 1, WN3 = WN * WN * WN;
     constexpr int WJ = T + 3, WJ3 = WJ * WJ * WJ;
     constexpr int MB = 54;   // species (<= 2) x 27 directions
+    constexpr int kLogT = T == 4 ? 2 : 3;
     // node e: sNa[e] = (Ex, Ey, Ez, Bx), sNb[e] = (By, Bz); 24 B per node keeps the LDS of a
     // tile-8 workgroup under a third of the CU's
     __shared__ float4 sNa[WN3];
@@ -290,7 +326,6 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
     __shared__ int sStart[MB + 1], sVs[MB];
     __shared__ unsigned sSrc[MB], sDstBase[MB];
     __shared__ int sDstCap[MB], sDstBin[MB], sCnt[MB];
-    __shared__ float sQm[4], sQs[4];
 
     const int tile = tile_remap(tp, blockIdx.x);
     const int tx = tile % tp.ntx, ty = (tile / tp.ntx) % tp.nty, tz = tile / (tp.ntx * tp.nty);
@@ -298,13 +333,16 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
     const int tid = threadIdx.x;
     const int mx = g.mx, nx = g.nx, ny = g.ny, nz = g.nz;
     const long long mxy = (long long)g.mx * g.my;
+    const bool edge = tx == 0 || ty == 0 || tz == 0 || tx == tp.ntx - 1 || ty == tp.nty - 1 || tz == tp.ntz - 1;
     const int nsp = tp.nsp, NV = nsp * 27;
 
+    int bcnt = 0;
     if (tid < NV) {
         // virtual bins: centre bins of every species first, then the 26 others
         int s, d;
         if (tid < nsp) { s = tid; d = 13; }
         else { const int r = tid - nsp; s = r / 26; const int q = r % 26; d = q < 13 ? q : q + 1; }
+        bcnt = bins.cnt_in[tile * tp.NB + s * 27 + d];
         sSrc[tid] = (unsigned)bins.base[tile * tp.NB + s * 27 + d];
         sVs[tid] = s;
         const int ds = tid / 27, dd = tid % 27;
@@ -317,18 +355,7 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
         sDstCap[tid] = bins.cap[db];
         sCnt[tid] = 0;
     }
-    if (tid == 0) {
-        int acc = 0;
-        for (int v = 0; v < NV; v++) {
-            int s, d;
-            if (v < nsp) { s = v; d = 13; }
-            else { const int r = v - nsp; s = r / 26; const int q = r % 26; d = q < 13 ? q : q + 1; }
-            sStart[v] = acc;
-            acc += bins.cnt_in[tile * tp.NB + s * 27 + d];
-        }
-        sStart[NV] = acc;
-        for (int s = 0; s < nsp; s++) { sQm[s] = (float)(ph.flvrqm[s] * 0.5); sQs[s] = (float)(ph.flvq[s] * kFixScale); }
-    }
+    if (tid < 64) bin_starts(bcnt, NV, sStart);
     const float bx0 = (float)ph.bext[0], by0 = (float)ph.bext[1], bz0 = (float)ph.bext[2];
     for (int e = tid; e < WN3; e += BS) {
         const int ii = e % WN, jj = (e / WN) % WN, kk = e / (WN * WN);
@@ -344,38 +371,52 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
 
     const float c = (float)ph.c, sqc = (float)ph.sqc, cinv = (float)ph.cinv;
     const float idx_ = (float)ph.inv_dx, idy_ = (float)ph.inv_dy, idz_ = (float)ph.inv_dz;
+    // q/m / 2 and the charge pre-scaled by 2^30 (exact) for the fixed-point current
+    const float qm0 = (float)(ph.flvrqm[0] * 0.5), qm1 = (float)(ph.flvrqm[1] * 0.5);
+    const float qs0 = (float)(ph.flvq[0] * kFixScale), qs1 = (float)(ph.flvq[1] * kFixScale);
     const int total = sStart[NV];
 
+    // position k lies in bin `bin` while k < binEnd, at slot k + binOff; a thread's k only grows
+    int bin = 0, binEnd = sStart[1], spc = sVs[0];
+    unsigned binOff = sSrc[0];
     auto load = [&](int k, SplitRec3 &r) {
-        const int v = bin_of<MB>(k, sStart, NV);
-        const unsigned off = (sSrc[v] + (unsigned)(k - sStart[v])) * 4u;
+        if (k >= binEnd) {
+            bin = bin_of<MB>(k, sStart, NV);
+            binEnd = sStart[bin + 1];
+            binOff = sSrc[bin] - (unsigned)sStart[bin];
+            spc = sVs[bin];
+        }
+        const unsigned off = (binOff + (unsigned)k) * 4u;
         r.cell = ldo(A.cell, off);
         r.ox = ldo(A.ox, off); r.oy = ldo(A.oy, off); r.oz = ldo(A.oz, off);
         r.u = ldo(A.u, off); r.v = ldo(A.v, off); r.w = ldo(A.w, off);
-        r.s = sVs[v];
         if (TAG) r.id = ldo(A.id, off);
         if (WQ) r.wq = ldo(A.wq, off);
     };
 
-    SplitRec3 nxt{};
-    if (tid < total) load(tid, nxt);
+    SplitRec3 cur;
+    if (tid < total) load(tid, cur);
+    settle(cur.cell, cur.ox, cur.oy, cur.oz, cur.u, cur.v, cur.w);
     for (int base = 0; base < total; base += BS) {
         const int k = base + tid;
         const bool active = k < total;
-        const SplitRec3 cur = nxt;
-        if (k + BS < total) load(k + BS, nxt);
-        int d = -1, ncell = cur.cell;
-        float ox = cur.ox, oy = cur.oy, oz = cur.oz, un = cur.u, vn = cur.v, wn = cur.w;
+        const int spn = spc;   // the species of `cur`
+        SplitRec3 nxt;
+        load(min(k + BS, total - 1), nxt);   // prefetch the next particle of this thread
+        int d = -1, ncell;
+        float ox, oy, oz, un, vn, wn;
         if (active) {
             int ci, cj, ck;
             cell_unpack(3, cur.cell, ci, cj, ck);
             const int gi = ci - (i0 - 3), gj = cj - (j0 - 3), gk = ck - (k0 - 3);   // 0..T-1 inside the tile
             if (gi < 0 || gi >= T || gj < 0 || gj >= T || gk < 0 || gk >= T) {
                 atomicOr(sp.err, (int)kErrBounds);
-                d = cur.s * 27 + 13;
+                d = spn * 27 + 13;
+                ncell = cur.cell;
+                ox = cur.ox; oy = cur.oy; oz = cur.oz; un = cur.u; vn = cur.v; wn = cur.w;
             } else {
                 const float x0 = cur.ox, y0 = cur.oy, z0 = cur.oz;
-                const float qm = sQm[cur.s], qs = WQ ? sQs[cur.s] * cur.wq : sQs[cur.s];
+                const float qm = spn ? qm1 : qm0, qsp = spn ? qs1 : qs0, qs = WQ ? qsp * cur.wq : qsp;
                 float wt[8];
 #pragma unroll
                 for (int cn = 0; cn < 8; cn++)
@@ -391,9 +432,9 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
                     hB[0] += wt[cn] * a.w; hB[1] += wt[cn] * b.x; hB[2] += wt[cn] * b.y;
                 }
                 const float pEx = pE[0] * qm, pEy = pE[1] * qm, pEz = pE[2] * qm;
-                float u0 = c * un + pEx;
-                float v0 = c * vn + pEy;
-                float w0 = c * wn + pEz;
+                float u0 = c * cur.u + pEx;
+                float v0 = c * cur.v + pEy;
+                float w0 = c * cur.w + pEz;
                 float gg = __builtin_amdgcn_rsqf(sqc + u0 * u0 + v0 * v0 + w0 * w0);
                 const float pBx = gg * hB[0] * qm, pBy = gg * hB[1] * qm, pBz = gg * hB[2] * qm;
                 const float f = 2.0f * __builtin_amdgcn_rcpf(1.0f + pBx * pBx + pBy * pBy + pBz * pBz);
@@ -412,60 +453,57 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
                 const float xr = fminf((float)(min(0, di) + 1), fmaxf((float)max(0, di), 0.5f * (x0 + x1)));
                 const float yr = fminf((float)(min(0, dj) + 1), fmaxf((float)max(0, dj), 0.5f * (y0 + y1)));
                 const float zr = fminf((float)(min(0, dk) + 1), fmaxf((float)max(0, dk), 0.5f * (z0 + z1)));
-                long long a[12], bq[12];
-#pragma unroll
-                for (int seg = 0; seg < 2; seg++) {
-                    const float Fx = seg ? qs * (x1 - xr) : qs * (xr - x0);
-                    const float Fy = seg ? qs * (y1 - yr) : qs * (yr - y0);
-                    const float Fz = seg ? qs * (z1 - zr) : qs * (zr - z0);
-                    const float Wx = seg ? 0.5f * (x1 + xr) - (float)di : 0.5f * (x0 + xr);
-                    const float Wy = seg ? 0.5f * (y1 + yr) - (float)dj : 0.5f * (y0 + yr);
-                    const float Wz = seg ? 0.5f * (z1 + zr) - (float)dk : 0.5f * (z0 + zr);
-                    long long *t = seg ? bq : a;
-                    t[0] = quanti((Fx * (1.0f - Wy)) * (1.0f - Wz)); t[1] = quanti((Fx * Wy) * (1.0f - Wz));
-                    t[2] = quanti((Fx * (1.0f - Wy)) * Wz);         t[3] = quanti((Fx * Wy) * Wz);
-                    t[4] = quanti((Fy * (1.0f - Wx)) * (1.0f - Wz)); t[5] = quanti((Fy * Wx) * (1.0f - Wz));
-                    t[6] = quanti((Fy * (1.0f - Wx)) * Wz);         t[7] = quanti((Fy * Wx) * Wz);
-                    t[8] = quanti((Fz * (1.0f - Wx)) * (1.0f - Wy)); t[9] = quanti((Fz * Wx) * (1.0f - Wy));
-                    t[10] = quanti((Fz * (1.0f - Wx)) * Wy);        t[11] = quanti((Fz * Wx) * Wy);
-                }
+                const float Fx[2] = {qs * (xr - x0), qs * (x1 - xr)};
+                const float Fy[2] = {qs * (yr - y0), qs * (y1 - yr)};
+                const float Fz[2] = {qs * (zr - z0), qs * (z1 - zr)};
+                const float Wx[2] = {0.5f * (x0 + xr), 0.5f * (x1 + xr) - (float)di};
+                const float Wy[2] = {0.5f * (y0 + yr), 0.5f * (y1 + yr) - (float)dj};
+                const float Wz[2] = {0.5f * (z0 + zr), 0.5f * (z1 + zr) - (float)dk};
                 const bool cross = (di != 0) || (dj != 0) || (dk != 0);
-                if (!cross) {
-#pragma unroll
-                    for (int q = 0; q < 12; q++) a[q] += bq[q];
-                }
                 constexpr int sy = WJ, sz = WJ * WJ;
-                {
-                    unsigned long long *jp = &sJ[0][((gk + 1) * WJ + (gj + 1)) * WJ + (gi + 1)];
-                    atomicAdd(jp, (unsigned long long)a[0]); atomicAdd(jp + sy, (unsigned long long)a[1]); atomicAdd(jp + sz, (unsigned long long)a[2]); atomicAdd(jp + sy + sz, (unsigned long long)a[3]);
-                    jp += WJ3;
-                    atomicAdd(jp, (unsigned long long)a[4]); atomicAdd(jp + 1, (unsigned long long)a[5]); atomicAdd(jp + sz, (unsigned long long)a[6]); atomicAdd(jp + 1 + sz, (unsigned long long)a[7]);
-                    jp += WJ3;
-                    atomicAdd(jp, (unsigned long long)a[8]); atomicAdd(jp + 1, (unsigned long long)a[9]); atomicAdd(jp + sy, (unsigned long long)a[10]); atomicAdd(jp + 1 + sy, (unsigned long long)a[11]);
-                }
-                if (cross) {
-                    unsigned long long *jp = &sJ[0][((gk + 1 + dk) * WJ + (gj + 1 + dj)) * WJ + (gi + 1 + di)];
-                    atomicAdd(jp, (unsigned long long)bq[0]); atomicAdd(jp + sy, (unsigned long long)bq[1]); atomicAdd(jp + sz, (unsigned long long)bq[2]); atomicAdd(jp + sy + sz, (unsigned long long)bq[3]);
-                    jp += WJ3;
-                    atomicAdd(jp, (unsigned long long)bq[4]); atomicAdd(jp + 1, (unsigned long long)bq[5]); atomicAdd(jp + sz, (unsigned long long)bq[6]); atomicAdd(jp + 1 + sz, (unsigned long long)bq[7]);
-                    jp += WJ3;
-                    atomicAdd(jp, (unsigned long long)bq[8]); atomicAdd(jp + 1, (unsigned long long)bq[9]); atomicAdd(jp + sy, (unsigned long long)bq[10]); atomicAdd(jp + 1 + sy, (unsigned long long)bq[11]);
-                }
+                const int ea = ((gk + 1) * WJ + (gj + 1)) * WJ + (gi + 1);
+                const int eb = ((gk + 1 + dk) * WJ + (gj + 1 + dj)) * WJ + (gi + 1 + di);
+                // F (1 - P, P) x (1 - Q, Q) on the nodes 0, sp, sq, sp + sq of a component, as counts;
+                // one component at a time keeps few of them in registers
+                auto deposit = [&](unsigned long long *w, const float *F, const float *P, const float *Q, int sp_, int sq_) {
+                    int v[2][4];
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const float l = F[h] * (1.0f - P[h]), u = F[h] * P[h];
+                        v[h][0] = quanti(l * (1.0f - Q[h])); v[h][1] = quanti(u * (1.0f - Q[h]));
+                        v[h][2] = quanti(l * Q[h]); v[h][3] = quanti(u * Q[h]);
+                    }
+                    long long t[4] = {v[0][0], v[0][1], v[0][2], v[0][3]};
+                    if (!cross) {
+#pragma unroll
+                        for (int m = 0; m < 4; m++) t[m] += v[1][m];
+                    }
+                    atomicAdd(w + ea, (unsigned long long)t[0]); atomicAdd(w + ea + sp_, (unsigned long long)t[1]);
+                    atomicAdd(w + ea + sq_, (unsigned long long)t[2]); atomicAdd(w + ea + sp_ + sq_, (unsigned long long)t[3]);
+                    if (cross) {
+                        atomicAdd(w + eb, (unsigned long long)(long long)v[1][0]);
+                        atomicAdd(w + eb + sp_, (unsigned long long)(long long)v[1][1]);
+                        atomicAdd(w + eb + sq_, (unsigned long long)(long long)v[1][2]);
+                        atomicAdd(w + eb + sp_ + sq_, (unsigned long long)(long long)v[1][3]);
+                    }
+                };
+                deposit(sJ[0], Fx, Wy, Wz, sy, sz);
+                deposit(sJ[1], Fy, Wx, Wz, 1, sz);
+                deposit(sJ[2], Fz, Wx, Wy, 1, sy);
                 ox = x1 - (float)di;
                 if (ox >= 1.0f) { ox = 0.0f; di += 1; }
                 oy = y1 - (float)dj;
                 if (oy >= 1.0f) { oy = 0.0f; dj += 1; }
                 oz = z1 - (float)dk;
                 if (oz >= 1.0f) { oz = 0.0f; dk += 1; }
-                int nci = ci + di, ncj = cj + dj, nck = ck + dk;
-                bool keep = true;
                 if (BC) {
                     // the boundary faces on the FP64 position; a reflected coordinate is
                     // split again into cell and offset
+                    int nci = ci + di, ncj = cj + dj, nck = ck + dk;
                     double X = 3.0 + (double)nci + (double)ox, Y = 3.0 + (double)ncj + (double)oy;
                     const double Z = 3.0 + (double)nck + (double)oz;
                     const double X0 = X, Y0 = Y;
-                    keep = particle_faces<float>(ph, g, X, Y, Z, un, vn);
+                    bool keep = particle_faces<float>(ph, g, X, Y, Z, un, vn);
                     if (keep && X != X0) {
                         const double f = floor(X);
                         nci = (int)f - 3;
@@ -481,19 +519,33 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
                     if ((nci < 0 || nci >= nx) && !g.per[0]) keep = false;
                     if ((ncj < 0 || ncj >= ny) && !g.per[1]) keep = false;
                     if ((nck < 0 || nck >= nz) && !g.per[2]) keep = false;
-                }
-                if (keep) {
-                    nci = nci < 0 ? nci + nx : (nci >= nx ? nci - nx : nci);
-                    ncj = ncj < 0 ? ncj + ny : (ncj >= ny ? ncj - ny : ncj);
-                    nck = nck < 0 ? nck + nz : (nck >= nz ? nck - nz : nck);
-                    ncell = cell_pack(3, nci, ncj, nck);
-                    const int ddx = norm_dir(nci / T - tx, tp.ntx), ddy = norm_dir(ncj / T - ty, tp.nty);
-                    const int ddz = norm_dir(nck / T - tz, tp.ntz);
-                    d = cur.s * 27 + (ddx + 1) + 3 * (ddy + 1) + 9 * (ddz + 1);
+                    if (keep) {
+                        nci = nci < 0 ? nci + nx : (nci >= nx ? nci - nx : nci);
+                        ncj = ncj < 0 ? ncj + ny : (ncj >= ny ? ncj - ny : ncj);
+                        nck = nck < 0 ? nck + nz : (nck >= nz ? nck - nz : nck);
+                        ncell = cell_pack(3, nci, ncj, nck);
+                        const int ddx = norm_dir(nci / T - tx, tp.ntx), ddy = norm_dir(ncj / T - ty, tp.nty);
+                        const int ddz = norm_dir(nck / T - tz, tp.ntz);
+                        d = spn * 27 + (ddx + 1) + 3 * (ddy + 1) + 9 * (ddz + 1);
+                    }
+                } else {
+                    // |di|, |dj|, |dk| <= 1: the destination is this tile or a neighbour, given by
+                    // the cell counted from the tile's corner (-1 .. T); only the tiles at the edge
+                    // of the box have cells to wrap
+                    ncell = cur.cell + di + dj * (1 << 11) + dk * (1 << 22);
+                    if (edge) {
+                        int nci = ci + di, ncj = cj + dj, nck = ck + dk;
+                        nci = nci < 0 ? nci + nx : (nci >= nx ? nci - nx : nci);
+                        ncj = ncj < 0 ? ncj + ny : (ncj >= ny ? ncj - ny : ncj);
+                        nck = nck < 0 ? nck + nz : (nck >= nz ? nck - nz : nck);
+                        ncell = cell_pack(3, nci, ncj, nck);
+                    }
+                    d = spn * 27 + 13 + ((gi + di) >> kLogT) + 3 * ((gj + dj) >> kLogT) + 9 * ((gk + dk) >> kLogT);
                 }
             }
         }
-        const int slot = reserve_slot(d, sCnt);
+        const int slot = reserve_slot(d, __builtin_amdgcn_readfirstlane(spn) * 27 + 13, sCnt);
+        settle(nxt.cell, nxt.ox, nxt.oy, nxt.oz, nxt.u, nxt.v, nxt.w);
         if (active && d >= 0) {
             if (slot < sDstCap[d]) {
                 const unsigned off = (sDstBase[d] + (unsigned)slot) * 4u;
@@ -505,7 +557,7 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
                 const int si = atomicAdd(sp.count, 1);
                 if (si < sp.cap) {
                     spill.cell[si] = ncell; spill.ox[si] = ox; spill.oy[si] = oy; spill.oz[si] = oz;
-                    spill.u[si] = un; spill.v[si] = vn; spill.w[si] = wn; spill.sp[si] = cur.s;
+                    spill.u[si] = un; spill.v[si] = vn; spill.w[si] = wn; spill.sp[si] = spn;
                     if (TAG) spill.id[si] = cur.id;
                     if (WQ) spill.wq[si] = cur.wq;
                 } else {
@@ -513,6 +565,7 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
                 }
             }
         }
+        cur = nxt;
     }
     __syncthreads();
     if (tid < NV) bins.cnt_out[sDstBin[tid]] = min(sCnt[tid], sDstCap[tid]);

@@ -33,24 +33,47 @@ __device__ inline int bin_of(int k, const int *sStart, int n)
     return b;
 }
 
-// Per-wave reservation of consecutive slots in the LDS counter of each
-// destination; every lane of the wave must call it (d = -1 for idle lanes).
-__device__ inline int reserve_slot(int d, int *sCnt)
+// Reservation of slots in the LDS counters of the destinations; every lane of the wave
+// must call it (d = -1 for idle lanes).  The lanes of the wave's usual destination `home`
+// (wave-uniform: the tile's own bin) take consecutive slots from one add by their first
+// lane; the few that leave the tile add for themselves, in the same LDS instruction.
+__device__ inline int reserve_slot(int d, int home, int *sCnt)
 {
-    const bool act = d >= 0;
-    unsigned long long pending = __ballot(act);
-    int slot = 0;
-    while (pending) {
-        const int leader = __ffsll((unsigned long long)pending) - 1;
-        const int ld = __shfl(d, leader);
-        const unsigned long long m = __ballot(act && d == ld);
-        int b = 0;
-        if ((int)__lane_id() == leader) b = atomicAdd(&sCnt[ld], __popcll(m));
-        b = __shfl(b, leader);
-        if (act && d == ld) slot = b + __popcll(m & lanemask_lt());
-        pending &= ~m;
+    const bool stay = d == home;
+    const unsigned long long m = __ballot(stay);
+    const unsigned rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+    int b = 0;
+    if (d >= 0 && (!stay || rank == 0u)) b = atomicAdd(&sCnt[d], stay ? __popcll(m) : 1);
+    const int b0 = __builtin_amdgcn_readlane(b, m ? __ffsll(m) - 1 : 0);
+    return stay ? b0 + (int)rank : b;
+}
+
+// a particle of the FP64 form as loaded
+struct RecF64 {
+    double x, y, z, u, v, w, q;
+    int flv, tag;
+};
+
+// Wait for the loads that fill `r`..., before the stores that follow in program order: loads
+// and stores share one counter, so a wait placed after them would last until they are done.
+template <typename... T>
+__device__ inline void settle(T &...r)
+{
+    (..., [](auto &v) { asm volatile("" : "+v"(v) : : "memory"); }(r));
+}
+
+// sStart[v] for v = 0..n from the counts `cnt` of the bins v = lane < n (n < 64), by one wave
+__device__ inline void bin_starts(int cnt, int n, int *sStart)
+{
+    const int lane = (int)__lane_id();
+    int acc = lane < n ? cnt : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int up = __shfl_up(acc, o);
+        if (lane >= o) acc += up;
     }
-    return slot;
+    if (lane < n) sStart[lane + 1] = acc;
+    if (lane == 0) sStart[0] = 0;
 }
 
 __device__ inline int wrap_tile(int t, int n)
@@ -67,45 +90,61 @@ __device__ inline int norm_dir(int dd, int n)
 
 // FP32 -> exact integer count of 2^-30 units (the argument is already scaled by 2^30;
 // |v| < 2^31, so one conversion)
-__device__ inline long long quanti(float v) { return (long long)(int)__builtin_rintf(v); }
+__device__ inline int quanti(float v) { return (int)__builtin_rintf(v); }
+
+// F * W as a count: rounded to the nearest integer (ties to even) by adding 1.5 * 2^52,
+// whose sum's bit pattern minus the constant's is that integer for |F W| < 2^51.
+constexpr double kCountBias = 6755399441055744.0;
+constexpr unsigned long long kCountBits = 0x4338000000000000ull;
+__device__ inline unsigned long long count_of(double F, double W)
+{
+    return (unsigned long long)__double_as_longlong(__builtin_fma(F, W, kCountBias)) - kCountBits;
+}
 
 // The two zigzag half-segments of the 2-D split form (movdep.F90:177-237)
-// from the old offsets (x0, y0, z0) to the new position as stored: offsets
-// (ox, oy) in the cell displaced by (di, dj), z advanced to z1.  Evaluated in
-// FP64, every relay point, flux F and weight W is exact for FP32 inputs and
-// each node value is rounded once before its rounding to a 2^-30 count, so
-// the deposited Jx, Jy carry exactly the charge moved between the stored
-// positions up to that last rounding.  qs: charge times 2^30.  a: the first
-// half-segment (nodes of the old cell), b: the second (nodes of the new cell),
-// each Jx (i,j), (i,j+1); Jy (i,j), (i+1,j); Jz (i,j), (i+1,j), (i,j+1), (i+1,j+1).
-__device__ inline void zigzag2d_split(double qs, float x0, float y0, float z0, float ox, float oy, float z1, int di,
-                                      int dj, double a[8], double b[8])
-{
-    const double X0 = x0, Y0 = y0, Z0 = z0;
-    const double X1 = (double)ox + (double)di, Y1 = (double)oy + (double)dj, Z1 = z1;
-    const int dk = (int)floor(Z1);
-    const double xr = dmin((double)(min(0, di) + 1), dmax((double)max(0, di), 0.5 * (X0 + X1)));
-    const double yr = dmin((double)(min(0, dj) + 1), dmax((double)max(0, dj), 0.5 * (Y0 + Y1)));
-    const double zr = dmin((double)(min(0, dk) + 1), dmax((double)max(0, dk), 0.5 * (Z0 + Z1)));
+// from the old offsets (x0, y0, kZMid) to the new position as stored: offsets
+// (ox, oy) in the cell displaced by (di, dj), each -1, 0 or 1, z advanced to z1.
+// Evaluated in FP64, every relay point, flux F and weight W is exact for FP32
+// inputs (F up to its product with the charge) and each node value is rounded
+// once to a 2^-30 count, so the deposited Jx, Jy carry exactly the charge moved
+// between the stored positions up to that last rounding.  qs: charge times 2^30.
+// Index 0: the first half-segment (nodes of the old cell), 1: the second (nodes
+// of the new cell).  The node counts are left to jx, jy, jz, so that a kernel
+// holds one component's at a time.
+struct Zigzag {
+    double Fx[2], Fy[2], Fz[2], Wx[2], Wy[2];
+
+    __device__ Zigzag(double qs, float x0, float y0, float ox, float oy, float z1, int di, int dj)
     {
-        const double Fx = qs * (xr - X0), Fy = qs * (yr - Y0), Fz = qs * (zr - Z0);
-        const double Wx = 0.5 * (X0 + xr), Wy = 0.5 * (Y0 + yr);
-        const double zl = Fz * (1.0 - Wx), zh = Fz * Wx;
-        a[0] = rint(Fx * (1.0 - Wy)); a[1] = rint(Fx * Wy);
-        a[2] = rint(Fy * (1.0 - Wx)); a[3] = rint(Fy * Wx);
-        a[4] = rint(zl * (1.0 - Wy)); a[5] = rint(zh * (1.0 - Wy));
-        a[6] = rint(zl * Wy); a[7] = rint(zh * Wy);
+        // relay point: the midpoint, or the face that was crossed
+        auto relay = [](double p0, double p1, int d) { return d == 0 ? 0.5 * (p0 + p1) : (d > 0 ? 1.0 : 0.0); };
+        const double X0 = x0, Y0 = y0, Z0 = kZMid;
+        const double dx = di, dy = dj;
+        const double X1 = (double)ox + dx, Y1 = (double)oy + dy, Z1 = z1;
+        const double xr = relay(X0, X1, di), yr = relay(Y0, Y1, dj);
+        const double zr = relay(Z0, Z1, z1 < 0.0f ? -1 : (z1 >= 1.0f ? 1 : 0));
+        Fx[0] = qs * (xr - X0); Fy[0] = qs * (yr - Y0); Fz[0] = qs * (zr - Z0);
+        Fx[1] = qs * (X1 - xr); Fy[1] = qs * (Y1 - yr); Fz[1] = qs * (Z1 - zr);
+        Wx[0] = 0.5 * (X0 + xr); Wy[0] = 0.5 * (Y0 + yr);
+        Wx[1] = __builtin_fma(0.5, X1 + xr, -dx); Wy[1] = __builtin_fma(0.5, Y1 + yr, -dy);
     }
+    // counts at (i, j), (i, j+1)
+    __device__ void jx(int h, unsigned long long n[2]) const
     {
-        const double Fx = qs * (X1 - xr), Fy = qs * (Y1 - yr), Fz = qs * (Z1 - zr);
-        const double Wx = 0.5 * (X1 + xr) - (double)di, Wy = 0.5 * (Y1 + yr) - (double)dj;
-        const double zl = Fz * (1.0 - Wx), zh = Fz * Wx;
-        b[0] = rint(Fx * (1.0 - Wy)); b[1] = rint(Fx * Wy);
-        b[2] = rint(Fy * (1.0 - Wx)); b[3] = rint(Fy * Wx);
-        b[4] = rint(zl * (1.0 - Wy)); b[5] = rint(zh * (1.0 - Wy));
-        b[6] = rint(zl * Wy); b[7] = rint(zh * Wy);
+        n[0] = count_of(Fx[h], 1.0 - Wy[h]); n[1] = count_of(Fx[h], Wy[h]);
     }
-}
+    // counts at (i, j), (i+1, j)
+    __device__ void jy(int h, unsigned long long n[2]) const
+    {
+        n[0] = count_of(Fy[h], 1.0 - Wx[h]); n[1] = count_of(Fy[h], Wx[h]);
+    }
+    // counts at (i, j), (i+1, j), (i, j+1), (i+1, j+1)
+    __device__ void jz(int h, unsigned long long n[4]) const
+    {
+        const double lo = Fz[h] * (1.0 - Wx[h]), hi = Fz[h] * Wx[h], Vy = 1.0 - Wy[h];
+        n[0] = count_of(lo, Vy); n[1] = count_of(hi, Vy); n[2] = count_of(lo, Wy[h]); n[3] = count_of(hi, Wy[h]);
+    }
+};
 
 // EnforceBC_PostMovDep (bc.F90:238-287) on one pushed particle, in the
 // reference's order: the reflecting faces top, bottom, right, left
