@@ -84,6 +84,9 @@ struct pictor_ctx {
     void *J[3] = {nullptr, nullptr, nullptr};
     // split form: the low FP32 part of E (E = hi + lo, hi in E[]), see launch_update_e_pair
     float *Elo[3] = {nullptr, nullptr, nullptr};
+    // second buffers of E, B, Elo and J: a fused step reads one set and writes the other
+    void *E2[3] = {nullptr, nullptr, nullptr}, *B2[3] = {nullptr, nullptr, nullptr}, *J2[3] = {nullptr, nullptr, nullptr};
+    float *Elo2[3] = {nullptr, nullptr, nullptr};
     // smoothen_current: passes per step and the filter's scratch current
     int curr_filter = 0;
     double *Jt[3] = {nullptr, nullptr, nullptr};
@@ -107,7 +110,8 @@ struct pictor_ctx {
     int spill_cap = 0;
     int *d_spill_count = nullptr;
     int *d_err = nullptr;
-    int *h_flags = nullptr;   // pinned: {spill count, error bits}
+    int *d_stop = nullptr;    // the first of several enqueued steps that spilled or failed (Gate)
+    int *h_flags = nullptr;   // pinned: {spill count, error bits, stop step}
     // re-layout scratch, allocated with the bins: per (tile, species) group counts,
     // totals, fill cursors and offsets; the group of each spilled particle
     int *rl_gcount = nullptr, *rl_gtotal = nullptr, *rl_fill = nullptr, *rl_grp = nullptr;
@@ -120,10 +124,12 @@ struct pictor_ctx {
     double *d_rho = nullptr;
 
     // timers: 0 push, 1 field kernels, 2 whole step.  ev[0..7]: the phase calls and the
-    // cylindrical steps; ev[8..14] and ev[15..21]: the fused Cartesian step, two sets of 7
-    // used alternately so that one step's events are read while the next step is being
-    // enqueued; ev[22]: the spill and error flags of a phase-call push copied to the host
+    // cylindrical steps; ev[8..14] and ev[15..21]: the fused step of a box with boundary faces,
+    // two sets of 7 used alternately so that one step's events are read while the next step is
+    // being enqueued; ev[22]: the spill and error flags of a phase-call push copied to the
+    // host; sev: before and after every push of a run of fused steps, and the run's end
     hipEvent_t ev[23] = {};
+    std::vector<hipEvent_t> sev;
     double t_ms[3] = {0, 0, 0};
     long long t_n[3] = {0, 0, 0};
 

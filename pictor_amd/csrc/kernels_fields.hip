@@ -174,14 +174,6 @@ __global__ __launch_bounds__(BX *BY) void k_update_e(GridP g, R fc, R idx_, R id
 // the curl terms cancels to FP64 rounding, and the fixed-point current
 // enters exactly scaled.  Everything that reads E for the push or the B
 // update reads hi, an ordinary FP32 field.
-// the value a double takes after being stored as an FP32 (hi, lo) pair and read back
-__device__ __forceinline__ double pair_round(double x)
-{
-    const float h = (float)x;
-    const float l = (float)(x - (double)h);
-    return (double)h + (double)l;
-}
-
 template <bool CURL, bool ADD>
 __global__ __launch_bounds__(BX *BY) void k_update_e_pair(GridP g, double fc, double idx_, double idy_, double idz_,
                                                           const float *__restrict__ Bx, const float *__restrict__ By,
@@ -217,7 +209,7 @@ __global__ __launch_bounds__(BX *BY) void k_update_e_pair(GridP g, double fc, do
         // round through the stored pair between the curl and the current, as the
         // separate UpdateEfield / AddCurrent phases do: the fused step and the
         // phase-by-phase host then give the same bits
-        ex = pair_round(ex); ey = pair_round(ey); ez = pair_round(ez);
+        ex = pair_value(ex); ey = pair_value(ey); ez = pair_value(ez);
     }
     if (ADD) {
         const bool inner = i >= 3 && i <= g.mx - 3 && j >= 3 && j <= g.my - 3 &&
@@ -286,8 +278,9 @@ __global__ __launch_bounds__(256) void k_ghost_copy(GridP g, Ptrs6<R> F)
 // UpdateCurrentAllFaces for one axis: 3..5 += m-2..m and m-4..m-3 += 1..2.
 // Axis 0 spans the full cross-section, axes 1 and 2 the x range 3..mx-3.
 template <typename JT>
-__global__ __launch_bounds__(256) void k_current_fold(GridP g, int axis, Ptrs6<JT> J)
+__global__ __launch_bounds__(256) void k_current_fold(GridP g, int axis, Ptrs6<JT> J, Gate gate)
 {
+    if (gate_closed(gate)) return;
     JT *__restrict__ J0 = J.p[3 * blockIdx.y];
     JT *__restrict__ J1 = J.p[3 * blockIdx.y + 1];
     JT *__restrict__ J2 = J.p[3 * blockIdx.y + 2];
@@ -327,8 +320,9 @@ __global__ __launch_bounds__(256) void k_current_fold(GridP g, int axis, Ptrs6<J
 // images (what SendRecvFldsYZ/ZX/XY put in the ghosts on one rank).  Every
 // other cell is copied, so dst is a complete array.  blockIdx.y selects the
 // component.
-__global__ __launch_bounds__(256) void k_filter_axis(GridP g, int axis, Ptrs6<double> P)
+__global__ __launch_bounds__(256) void k_filter_axis(GridP g, int axis, Ptrs6<double> P, Gate gate)
 {
+    if (gate_closed(gate)) return;
     const double *__restrict__ src = P.p[blockIdx.y];
     double *__restrict__ dst = P.p[3 + blockIdx.y];
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -363,8 +357,9 @@ __global__ __launch_bounds__(256) void k_fill_zero(Ptrs6<T> P, long long n)
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_copy_n(Ptrs6<T> D, Ptrs6<T> S, long long n)
+__global__ __launch_bounds__(256) void k_copy_n(Ptrs6<T> D, Ptrs6<T> S, long long n, Gate gate)
 {
+    if (gate_closed(gate)) return;
     T *d = D.p[blockIdx.y];
     const T *src = S.p[blockIdx.y];
     long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -518,7 +513,7 @@ void launch_ghost_copy(const GridP &g, R *const F[3], hipStream_t s, R *const G[
 }
 
 template <typename JT>
-void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, JT *const K[3])
+void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, JT *const K[3], Gate gate)
 {
     Ptrs6<JT> P{{J[0], J[1], J[2], K ? K[0] : nullptr, K ? K[1] : nullptr, K ? K[2] : nullptr}};
     int naxes = (g.ndim == 3) ? 3 : 2;
@@ -528,11 +523,11 @@ void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, JT *cons
         if (a != 0) ext[0] = g.mx - 5;
         ext[a] = 5;
         long long total = ext[0] * ext[1] * ext[2];
-        hipLaunchKernelGGL(k_current_fold<JT>, dim3(nblocks(total, 256), K ? 2 : 1), dim3(256), 0, s, g, a, P);
+        hipLaunchKernelGGL(k_current_fold<JT>, dim3(nblocks(total, 256), K ? 2 : 1), dim3(256), 0, s, g, a, P, gate);
     }
 }
 
-void launch_smoothen_current(const GridP &g, int passes, double *const J[3], double *const T[3], hipStream_t s)
+void launch_smoothen_current(const GridP &g, int passes, double *const J[3], double *const T[3], hipStream_t s, Gate gate)
 {
     const int naxes = (g.ndim == 3) ? 3 : 2;
     Ptrs6<double> fwd{{J[0], J[1], J[2], T[0], T[1], T[2]}}, back{{T[0], T[1], T[2], J[0], J[1], J[2]}};
@@ -540,10 +535,10 @@ void launch_smoothen_current(const GridP &g, int passes, double *const J[3], dou
     for (int ni = 0; ni < passes; ni++)
         for (int a = 0; a < naxes; a++) {
             hipLaunchKernelGGL(k_filter_axis, dim3(nblocks(g.ncell, 256), 3), dim3(256), 0, s, g, a,
-                               in_t ? back : fwd);
+                               in_t ? back : fwd, gate);
             in_t = !in_t;
         }
-    if (in_t) launch_copy_n<double>(J, T, 3, g.ncell, s);
+    if (in_t) launch_copy_n<double>(J, T, 3, g.ncell, s, gate);
 }
 
 template <typename T>
@@ -564,14 +559,14 @@ void launch_fill_zero(T *p, long long n, hipStream_t s)
 }
 
 template <typename T>
-void launch_copy_n(T *const *dst, T *const *src, int count, long long n, hipStream_t s)
+void launch_copy_n(T *const *dst, T *const *src, int count, long long n, hipStream_t s, Gate gate)
 {
     unsigned nb = nblocks(n, 256);
     if (nb > 65536u) nb = 65536u;
     if (nb == 0 || count < 1) return;
     Ptrs6<T> D{}, S{};
     for (int i = 0; i < count && i < 6; i++) { D.p[i] = dst[i]; S.p[i] = src[i]; }
-    hipLaunchKernelGGL(k_copy_n<T>, dim3(nb, count < 6 ? count : 6), dim3(256), 0, s, D, S, n);
+    hipLaunchKernelGGL(k_copy_n<T>, dim3(nb, count < 6 ? count : 6), dim3(256), 0, s, D, S, n, gate);
 }
 
 template <typename R>
@@ -653,11 +648,11 @@ template void launch_add_current<float, double>(const GridP &, const PhysP &, fl
                                                 double, hipStream_t);
 template void launch_ghost_copy<double>(const GridP &, double *const[3], hipStream_t, double *const[3]);
 template void launch_ghost_copy<float>(const GridP &, float *const[3], hipStream_t, float *const[3]);
-template void launch_current_fold<double>(const GridP &, double *const[3], hipStream_t, double *const[3]);
+template void launch_current_fold<double>(const GridP &, double *const[3], hipStream_t, double *const[3], Gate);
 template void launch_fill_zero_n<double>(double *const *, int, long long, hipStream_t);
 template void launch_fill_zero_n<float>(float *const *, int, long long, hipStream_t);
-template void launch_copy_n<float>(float *const *, float *const *, int, long long, hipStream_t);
-template void launch_copy_n<double>(double *const *, double *const *, int, long long, hipStream_t);
+template void launch_copy_n<float>(float *const *, float *const *, int, long long, hipStream_t, Gate);
+template void launch_copy_n<double>(double *const *, double *const *, int, long long, hipStream_t, Gate);
 template void launch_fill_zero<double>(double *, long long, hipStream_t);
 template void launch_fill_zero<float>(float *, long long, hipStream_t);
 template void launch_fill_zero<long long>(long long *, long long, hipStream_t);

@@ -59,6 +59,7 @@ __global__ __launch_bounds__(BS) void k_push2d_f64(GridP g, PhysP ph, TileP tp, 
     __shared__ long long sDstBase[9];
     __shared__ int sDstCap[9], sDstBin[9], sCnt[9];
 
+    if (sp.stop && *sp.stop < sp.step) return;
     const int tile = tile_remap(tp, blockIdx.x);
     const int tx = tile % tp.ntx, ty = tile / tp.ntx;
     const int iw = 1 + tx * T, jw = 1 + ty * T;   // window origin = first cell - 2 (reference index)
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(BS) void k_push2d_f64(GridP g, PhysP ph, TileP tp, 
             const int ii0 = ip0 - iw, jj0 = jp0 - jw;
             xn = x0; yn = y0; zn = z0;
             if (ii0 < 1 || ii0 > W - 3 || jj0 < 1 || jj0 > W - 3 || flv < 1 || flv > ph.nflvr) {
-                atomicOr(sp.err, (int)kErrBounds);
+                flag_error(sp, kErrBounds);
                 d = 4;
             } else {
                 // gather, movdep.F90:88-139
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(BS) void k_push2d_f64(GridP g, PhysP ph, TileP tp, 
                     cy = cy < 0 ? 0 : (cy > g.ny - 1 ? g.ny - 1 : cy);
                     const int ddx = norm_dir(cx / T - tx, tp.ntx), ddy = norm_dir(cy / T - ty, tp.nty);
                     if (ddx < -1 || ddx > 1 || ddy < -1 || ddy > 1) {
-                        atomicOr(sp.err, (int)kErrBounds);
+                        flag_error(sp, kErrBounds);
                         d = 4;
                     } else {
                         d = (ddx + 1) + 3 * (ddy + 1);
@@ -271,14 +272,14 @@ __global__ __launch_bounds__(BS) void k_push2d_f64(GridP g, PhysP ph, TileP tp, 
                 Bo.q[o] = q; Bo.flv[o] = flv;
                 if (TAG) Bo.tag[o] = tg;
             } else {
-                const int s = atomicAdd(sp.count, 1);
+                const int s = spill_slot(sp);
                 if (s < sp.cap) {
                     spill.x[s] = xn; spill.y[s] = yn; spill.z[s] = zn;
                     spill.u[s] = un; spill.v[s] = vn; spill.w[s] = wn;
                     spill.q[s] = q; spill.flv[s] = flv;
                     if (TAG) spill.tag[s] = tg;
                 } else {
-                    atomicOr(sp.err, (int)kErrCapacity);
+                    flag_error(sp, kErrCapacity);
                 }
             }
         }
@@ -343,6 +344,7 @@ __global__ __launch_bounds__(BS) void k_push2d_split(GridP g, PhysP ph, TileP tp
     __shared__ unsigned sSrc[MB], sDstBase[MB];
     __shared__ int sDstCap[MB], sDstBin[MB], sCnt[MB];
 
+    if (sp.stop && *sp.stop < sp.step) return;
     const int tile = tile_remap(tp, blockIdx.x);
     const int tx = tile % tp.ntx, ty = tile / tp.ntx;
     const int iw = 1 + tx * T, jw = 1 + ty * T;
@@ -436,7 +438,7 @@ __global__ __launch_bounds__(BS) void k_push2d_split(GridP g, PhysP ph, TileP tp
             const int ci = cur.cell & 0xFFFF, cj = cur.cell >> 16;
             const int ii0 = ci - cx0, jj0 = cj - cy0;
             if (ii0 < 2 || ii0 > T + 1 || jj0 < 2 || jj0 > T + 1) {
-                atomicOr(sp.err, (int)kErrBounds);
+                flag_error(sp, kErrBounds);
                 d = spn * 9 + 4;
                 ncell = cur.cell;
                 ox = cur.ox; oy = cur.oy; un = cur.u; vn = cur.v; wn = cur.w;
@@ -559,14 +561,14 @@ __global__ __launch_bounds__(BS) void k_push2d_split(GridP g, PhysP ph, TileP tp
                 if (WQ) sto(Bo.wq, off, cur.wq);
                 if (TRACK && dst) dst[cur.slot] = (int)(sDstBase[d] + (unsigned)slot);
             } else {
-                const int si = atomicAdd(sp.count, 1);
+                const int si = spill_slot(sp);
                 if (si < sp.cap) {
                     spill.cell[si] = ncell; spill.ox[si] = ox; spill.oy[si] = oy;
                     spill.u[si] = un; spill.v[si] = vn; spill.w[si] = wn; spill.sp[si] = spn;
                     if (TAG) spill.id[si] = cur.id;
                     if (WQ) spill.wq[si] = cur.wq;
                 } else {
-                    atomicOr(sp.err, (int)kErrCapacity);
+                    flag_error(sp, kErrCapacity);
                 }
                 if (TRACK && dst) dst[cur.slot] = -1;
             }
@@ -586,7 +588,7 @@ __global__ __launch_bounds__(BS) void k_push2d_split(GridP g, PhysP ph, TileP tp
         if (b != 0.0) unsafeAtomicAdd(&Jy[o], b);
         if (cz != 0.0) unsafeAtomicAdd(&Jz[o], cz);
     }
-    if (big) atomicOr(sp.err, (int)kErrPrecision);
+    if (big) flag_error(sp, kErrPrecision);
 }
 
 }  // namespace

@@ -39,6 +39,7 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
     __shared__ long long sSrc[27], sDstBase[27];
     __shared__ int sDstCap[27], sDstBin[27], sCnt[27];
 
+    if (sp.stop && *sp.stop < sp.step) return;
     const int tile = tile_remap(tp, blockIdx.x);
     const int tx = tile % tp.ntx, ty = (tile / tp.ntx) % tp.nty, tz = tile / (tp.ntx * tp.nty);
     const int i0 = 3 + tx * T, j0 = 3 + ty * T, k0 = 3 + tz * T;   // first cell of the tile
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
             // node-window coordinates of the cell (origin i0-1)
             const int gi = ip0 - (i0 - 1), gj = jp0 - (j0 - 1), gk = kp0 - (k0 - 1);
             if (gi < 0 || gi > T + 1 || gj < 0 || gj > T + 1 || gk < 0 || gk > T + 1 || flv < 1 || flv > ph.nflvr) {
-                atomicOr(sp.err, (int)kErrBounds);
+                flag_error(sp, kErrBounds);
                 d = 13;
             } else {
                 const double dx = x0 - ip0, dy = y0 - jp0, dz = z0 - kp0;
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
                     const int ddx = norm_dir(cx / T - tx, tp.ntx), ddy = norm_dir(cy / T - ty, tp.nty);
                     const int ddz = norm_dir(cz / T - tz, tp.ntz);
                     if (ddx < -1 || ddx > 1 || ddy < -1 || ddy > 1 || ddz < -1 || ddz > 1) {
-                        atomicOr(sp.err, (int)kErrBounds);
+                        flag_error(sp, kErrBounds);
                         d = 13;
                     } else {
                         d = (ddx + 1) + 3 * (ddy + 1) + 9 * (ddz + 1);
@@ -270,14 +271,14 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
                 Bo.q[o] = q; Bo.flv[o] = flv;
                 if (TAG) Bo.tag[o] = tg;
             } else {
-                const int s = atomicAdd(sp.count, 1);
+                const int s = spill_slot(sp);
                 if (s < sp.cap) {
                     spill.x[s] = xn; spill.y[s] = yn; spill.z[s] = zn;
                     spill.u[s] = un; spill.v[s] = vn; spill.w[s] = wn;
                     spill.q[s] = q; spill.flv[s] = flv;
                     if (TAG) spill.tag[s] = tg;
                 } else {
-                    atomicOr(sp.err, (int)kErrCapacity);
+                    flag_error(sp, kErrCapacity);
                 }
             }
         }
@@ -327,6 +328,7 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
     __shared__ unsigned sSrc[MB], sDstBase[MB];
     __shared__ int sDstCap[MB], sDstBin[MB], sCnt[MB];
 
+    if (sp.stop && *sp.stop < sp.step) return;
     const int tile = tile_remap(tp, blockIdx.x);
     const int tx = tile % tp.ntx, ty = (tile / tp.ntx) % tp.nty, tz = tile / (tp.ntx * tp.nty);
     const int i0 = 3 + tx * T, j0 = 3 + ty * T, k0 = 3 + tz * T;
@@ -410,7 +412,7 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
             cell_unpack(3, cur.cell, ci, cj, ck);
             const int gi = ci - (i0 - 3), gj = cj - (j0 - 3), gk = ck - (k0 - 3);   // 0..T-1 inside the tile
             if (gi < 0 || gi >= T || gj < 0 || gj >= T || gk < 0 || gk >= T) {
-                atomicOr(sp.err, (int)kErrBounds);
+                flag_error(sp, kErrBounds);
                 d = spn * 27 + 13;
                 ncell = cur.cell;
                 ox = cur.ox; oy = cur.oy; oz = cur.oz; un = cur.u; vn = cur.v; wn = cur.w;
@@ -554,14 +556,14 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
                 if (TAG) sto(Bo.id, off, cur.id);
                 if (WQ) sto(Bo.wq, off, cur.wq);
             } else {
-                const int si = atomicAdd(sp.count, 1);
+                const int si = spill_slot(sp);
                 if (si < sp.cap) {
                     spill.cell[si] = ncell; spill.ox[si] = ox; spill.oy[si] = oy; spill.oz[si] = oz;
                     spill.u[si] = un; spill.v[si] = vn; spill.w[si] = wn; spill.sp[si] = spn;
                     if (TAG) spill.id[si] = cur.id;
                     if (WQ) spill.wq[si] = cur.wq;
                 } else {
-                    atomicOr(sp.err, (int)kErrCapacity);
+                    flag_error(sp, kErrCapacity);
                 }
             }
         }
@@ -580,7 +582,7 @@ __global__ __launch_bounds__(BS) void k_push3d_split(GridP g, PhysP ph, TileP tp
         if (b != 0.0) unsafeAtomicAdd(&Jy[o], b);
         if (cz != 0.0) unsafeAtomicAdd(&Jz[o], cz);
     }
-    if (big) atomicOr(sp.err, (int)kErrPrecision);
+    if (big) flag_error(sp, kErrPrecision);
 }
 
 }  // namespace

@@ -141,6 +141,23 @@ __device__ inline int tile_remap(const TileP &tp, int bid)
     return (bid & 7) * per + (bid >> 3);
 }
 
+// Launches of several steps are enqueued before the host looks at the first one's flags: a
+// kernel of a step after `*stop` returns at once (stop null: always open).
+constexpr int kNoStop = 0x7f7f7f7f;   // four equal bytes: set with a memset
+struct Gate {
+    const int *stop = nullptr;
+    int step = 0;
+};
+__device__ inline bool gate_closed(const Gate &g) { return g.stop && *g.stop < g.step; }
+
+// the value a double takes after being stored as an FP32 (hi, lo) pair and read back
+__device__ __forceinline__ double pair_value(double x)
+{
+    const float h = (float)x;
+    const float l = (float)(x - (double)h);
+    return (double)h + (double)l;
+}
+
 // ---------------- launchers (kernels_fields.hip) ----------------
 template <typename R>
 void launch_update_b_half(const GridP &g, const PhysP &ph, R *const E[3], R *const B[3], hipStream_t s);
@@ -167,16 +184,17 @@ struct Ptrs6 {
 template <typename R>
 void launch_ghost_copy(const GridP &g, R *const F[3], hipStream_t s, R *const G[3] = nullptr);
 template <typename JT>
-void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, JT *const K[3] = nullptr);
+void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, JT *const K[3] = nullptr, Gate gate = Gate{});
 template <typename T>
 void launch_fill_zero(T *p, long long n, hipStream_t s);
 template <typename T>
 void launch_fill_zero_n(T *const *p, int count, long long n, hipStream_t s);   // count <= 6
 template <typename T>
-void launch_copy_n(T *const *dst, T *const *src, int count, long long n, hipStream_t s);   // count <= 6
+void launch_copy_n(T *const *dst, T *const *src, int count, long long n, hipStream_t s, Gate gate = Gate{});   // count <= 6
 // smoothen_current: `passes` rounds of the 1-2-1 filter along each axis, J in
 // place, T (three arrays of ncell) as scratch
-void launch_smoothen_current(const GridP &g, int passes, double *const J[3], double *const T[3], hipStream_t s);
+void launch_smoothen_current(const GridP &g, int passes, double *const J[3], double *const T[3], hipStream_t s,
+                             Gate gate = Gate{});
 template <typename R>
 void launch_field_energy(const GridP &g, R *const E[3], R *const B[3], double *partial, int nblk, hipStream_t s,
                          R *const *L = nullptr);
@@ -204,6 +222,10 @@ struct SpillP {
     int *count;
     int cap;
     int *err;
+    // the first step that spilled or failed, among steps enqueued together (null: none are);
+    // a push of a later step does nothing
+    int *stop = nullptr;
+    int step = 0;
 };
 
 void launch_push2d_f64(int T, const GridP &g, const PhysP &ph, const TileP &tp, double *const E[3],

@@ -14,6 +14,18 @@ __device__ inline unsigned long long lanemask_lt()
     return (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
 }
 
+// an error of this step, and a spilled particle: both stop the steps enqueued behind it
+__device__ inline void flag_error(const SpillP &sp, int bits)
+{
+    atomicOr(sp.err, bits);
+    if (sp.stop) atomicMin(sp.stop, sp.step);
+}
+__device__ inline int spill_slot(const SpillP &sp)
+{
+    if (sp.stop) atomicMin(sp.stop, sp.step);
+    return atomicAdd(sp.count, 1);
+}
+
 // Bin of position k (0 <= k < sStart[n]) among n bins laid end to end: the last b < n with
 // sStart[b] <= k (an empty bin shares its start with the next).  A search of fixed depth (5 or 6
 // LDS reads) for the 27-direction bins of the 3-D layout, where a linear walk from the first bin
