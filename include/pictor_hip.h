@@ -286,12 +286,12 @@ int pictor_adjoint_forward_device(pictor_ctx *ctx, int64_t n, const double *q, c
                                   double *objective);
 int pictor_adjoint_backward_device(pictor_ctx *ctx, double scale, double *du, double *dv, double *dw);
 int pictor_adjoint_stats(pictor_ctx *ctx, double out[10]);
-/* Engine of the FP32 split form: 0 = tile-sorted (default; the particles in
- * the tile bins of pictor_move_deposit, every forward step the production
- * push, the reverse step over the same bins with LDS gather and LDS
- * accumulation of the field adjoint; tile edge 8, 16 or 32), 1 = unsorted
- * (one thread per particle, global atomics).  The FP64 form always uses the
- * unsorted engine.  Takes effect at the next pictor_adjoint_forward. */
+/* Engine: 0 = tile-sorted (default; the particles in tile bins, the field and
+ * the current of a tile in LDS, the reverse step over the same bins; FP32 split
+ * form: every forward step the production push, tile edge 8, 16 or 32; FP64:
+ * tile edge 8 or 16 and memory for the bins of every kept state, otherwise the
+ * unsorted engine), 1 = unsorted (one thread per particle, global atomics).
+ * Takes effect at the next pictor_adjoint_forward. */
 int pictor_adjoint_engine(pictor_ctx *ctx, int32_t engine);
 int pictor_adjoint_release(pictor_ctx *ctx);
 

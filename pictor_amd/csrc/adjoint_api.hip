@@ -7,11 +7,13 @@
 // then runs the reverse steps of that segment.
 //
 // Two engines:
-//  * tile-sorted (FP32 split form only): the particles live in the
-//    production tile bins and every forward step is the production push
-//    kernel in its index-carrying variant, which also records for every
-//    input slot the slot its particle went to.  The reverse step walks the
-//    same bins (adjoint_fast.hip).  Recomputed states hold the same particles
+//  * tile-sorted: the particles live in tile bins.  FP32: the production bins,
+//    every forward step the production push kernel in its index-carrying
+//    variant; FP64 (tile 8 or 16, where its states fit in memory): k_fa_push64.
+//    The push records for every input slot the slot its particle went to, and
+//    the reverse step walks the same bins (adjoint_fast.hip).  The field work of
+//    a step is one launch (kernels_fieldstep.hip), which writes the E and B that
+//    the next push reads straight into the arrays the reverse sweep keeps.  Recomputed states hold the same particles
 //    as the forward pass's, possibly in another order inside a bin (slot
 //    reservation order varies between runs); the particle ids map the
 //    adjoint from one to the other at segment boundaries.
@@ -24,6 +26,7 @@
 
 #include "adjoint.h"
 #include "ctx.h"
+#include "fieldstep.h"
 
 using namespace pictor;
 
@@ -31,6 +34,7 @@ namespace {
 
 constexpr double kFixQ = kFixScale;   // the split form's current counts per charge cell
 constexpr int kRetryLayout = -100;   // internal: tile bins overflowed, redo with larger bins
+constexpr int kUseUnsorted = -101;   // internal: the FP64 tile bins do not fit, use the unsorted engine
 
 template <typename R>
 hipError_t alloc_part(EPart<R> &p, long long n, long long &bytes, bool with_cs = true)
@@ -65,7 +69,7 @@ hipError_t copy_part(EPart<R> dst, EPart<R> src, long long n, hipStream_t s)
 }
 
 // split-form particle storage of `cap` slots: with_id for the engine's states, with_sp for the spill buffer
-hipError_t alloc_split_state(PartSplit &p, long long cap, bool with_id, bool with_sp, long long &bytes)
+hipError_t alloc_state(PartSplit &p, long long cap, bool with_id, bool with_sp, long long &bytes)
 {
     hipError_t e;
     p = PartSplit{};
@@ -80,7 +84,22 @@ hipError_t alloc_split_state(PartSplit &p, long long cap, bool with_id, bool wit
     return hipSuccess;
 }
 
-void free_split_state(PartSplit &p)
+hipError_t alloc_state(PartE64 &p, long long cap, bool, bool, long long &bytes)
+{
+    hipError_t e = alloc_part(p.p, cap, bytes);
+    if (e == hipSuccess) e = dalloc(&p.id, cap);
+    bytes += 4 * cap;
+    return e;
+}
+
+void free_state(PartE64 &p)
+{
+    free_part(p.p);
+    dfree(p.id);
+    p = PartE64{};
+}
+
+void free_state(PartSplit &p)
 {
     dfree(p.cell); dfree(p.ox); dfree(p.oy); dfree(p.oz); dfree(p.u); dfree(p.v); dfree(p.w);
     dfree(p.id); dfree(p.sp);
@@ -165,7 +184,7 @@ struct AdjEngine : AdjEngineBase {
     std::vector<void *> nodE, nodB;     // node fields of one segment (seg)
     EPart<R> adj{};
 
-    // tile-sorted engine (R = float): the production tile bins
+    // tile-sorted engine: the tile bins
     bool fast = false;
     double cap_factor = 1.5;            // centre-bin capacity / particles of the group at load time
     int relayouts = 0;                  // forward passes repeated with larger bins
@@ -174,13 +193,17 @@ struct AdjEngine : AdjEngineBase {
     long long lay_total = 0;
     long long *d_base = nullptr;
     int *d_cap = nullptr;
-    std::vector<PartSplit> ck2;         // particle checkpoints (nseg)
+    using State = typename FaState<R>::T;
+    std::vector<State> ck2;             // particle checkpoints (nseg)
     std::vector<int *> ck_cnt;          // their bin counts
-    std::vector<PartSplit> st2;         // states 1.. of a segment
+    std::vector<State> st2;             // states 1.. of a segment
     std::vector<int *> cntv;            // their bin counts
     std::vector<int *> dstv;            // per step of a segment: output slot of every input slot
-    std::vector<float *> sfE, sfB;      // per step of a segment: E and B as the push saw them
-    EPart<float> fa[2] = {};            // particle adjoints, indexed by slot
+    std::vector<R *> sfE, sfB;          // per step of a segment: E and B as the push saw them
+    R *E2[3] = {}, *B2[3] = {};         // second buffers of E, B, Elo and J
+    float *Elo2[3] = {};
+    double *J2[3] = {};
+    EPart<R> fa[2] = {};            // particle adjoints, indexed by slot
     int *pos = nullptr;                 // particle id -> slot
     PartSplit spill{};
     int spill_cap = 0;
@@ -210,18 +233,22 @@ struct AdjEngine : AdjEngineBase {
         for (void *p : nodB) dfree(p);
         nodE.clear(); nodB.clear();
         free_part(adj);
-        for (auto &p : ck2) free_split_state(p);
-        for (auto &p : st2) free_split_state(p);
+        for (auto &p : ck2) free_state(p);
+        for (auto &p : st2) free_state(p);
         ck2.clear(); st2.clear();
         for (int *p : ck_cnt) dfree(p);
         for (int *p : cntv) dfree(p);
         for (int *p : dstv) dfree(p);
         ck_cnt.clear(); cntv.clear(); dstv.clear();
-        for (float *p : sfE) dfree(p);
-        for (float *p : sfB) dfree(p);
+        for (R *p : sfE) dfree(p);
+        for (R *p : sfB) dfree(p);
         sfE.clear(); sfB.clear();
+        for (int i = 0; i < 3; i++) {
+            dfree(E2[i]); dfree(B2[i]); dfree(Elo2[i]); dfree(J2[i]);
+            E2[i] = B2[i] = nullptr; Elo2[i] = nullptr; J2[i] = nullptr;
+        }
         free_part(fa[0]); free_part(fa[1]);
-        free_split_state(spill);
+        free_state(spill);
         dfree(d_base); dfree(d_cap); dfree(pos); dfree(d_spill);
         d_base = nullptr; d_cap = nullptr; pos = nullptr; d_spill = nullptr;
         h_base.clear(); h_cap.clear();
@@ -237,7 +264,7 @@ struct AdjEngine : AdjEngineBase {
     {
         release();
         c = ctx;
-        fast = use_fast && std::is_same<R, float>::value;
+        fast = use_fast && (std::is_same<R, float>::value || ctx->tp.T == 8 || ctx->tp.T == 16);
         cap_factor = cf;
         n = np; nsteps = ns; seg = sg;
         nseg = (nsteps + seg - 1) / seg;
@@ -305,18 +332,18 @@ struct AdjEngine : AdjEngineBase {
         HIPTRY(dalloc(&d_cap, nb));
         HIPTRY(hipMemcpyAsync(d_base, h_base.data(), nb * sizeof(long long), hipMemcpyHostToDevice, c->stream));
         HIPTRY(hipMemcpyAsync(d_cap, h_cap.data(), nb * sizeof(int), hipMemcpyHostToDevice, c->stream));
-        ck2.assign(nseg, PartSplit{});
+        ck2.assign(nseg, State{});
         ck_cnt.assign(nseg, nullptr);
         for (int k = 0; k < nseg; k++) {
-            HIPTRY(alloc_split_state(ck2[k], lay_total, true, false, bytes));
+            HIPTRY(alloc_state(ck2[k], lay_total, true, false, bytes));
             HIPTRY(dalloc(&ck_cnt[k], nb));
         }
         // states 1..seg of a segment; the first pass ping-pongs between 1 and 2
         const int ns = std::max(seg, 2) + 1;
-        st2.assign(ns, PartSplit{});
+        st2.assign(ns, State{});
         cntv.assign(ns, nullptr);
         for (int j = 1; j < ns; j++) {
-            HIPTRY(alloc_split_state(st2[j], lay_total, true, false, bytes));
+            HIPTRY(alloc_state(st2[j], lay_total, true, false, bytes));
             HIPTRY(dalloc(&cntv[j], nb));
         }
         dstv.assign(seg, nullptr);
@@ -327,14 +354,21 @@ struct AdjEngine : AdjEngineBase {
             HIPTRY(dalloc(&sfE[i], ncell));
             HIPTRY(dalloc(&sfB[i], ncell));
         }
+        for (int i = 0; i < 3; i++) {
+            HIPTRY(dalloc(&E2[i], ncell)); HIPTRY(dalloc(&B2[i], ncell)); HIPTRY(dalloc(&J2[i], ncell));
+            if (Elo[i]) HIPTRY(dalloc(&Elo2[i], ncell));
+        }
+        bytes += ncell * (6 * (long long)sizeof(R) + 24 + (Elo[0] ? 12 : 0));
         HIPTRY(alloc_part(fa[0], lay_total, bytes, false));
         HIPTRY(alloc_part(fa[1], lay_total, bytes, false));
         HIPTRY(dalloc(&pos, n));
-        spill_cap = 4096;
-        HIPTRY(alloc_split_state(spill, spill_cap, false, true, bytes));
+        if constexpr (std::is_same<R, float>::value) {
+            spill_cap = 4096;
+            HIPTRY(alloc_state(spill, spill_cap, false, true, bytes));
+        }
         HIPTRY(dalloc(&d_spill, 1));
         bytes += (long long)(nseg + ns) * 4 * nb + 12LL * nb + (long long)seg * 4 * lay_total +
-                 (long long)seg * 24 * ncell + 4 * n;
+                 (long long)seg * 6 * sizeof(R) * ncell + 4 * n;
         return PICTOR_OK;
     }
 
@@ -396,22 +430,33 @@ struct AdjEngine : AdjEngineBase {
         long long *d_off = nullptr;
         auto cleanup = [&]() {
             (void)hipStreamSynchronize(s);
-            for (auto p : ds) dfree(*p);
-            dfree(raw.flv); dfree(d_tile); dfree(d_count); dfree(d_fill); dfree(d_off);
+            if (kin == hipMemcpyHostToDevice) {
+                for (auto p : ds) dfree(*p);
+                dfree(raw.flv);
+            }
+            dfree(d_tile); dfree(d_count); dfree(d_fill); dfree(d_off);
         };
         int rc = PICTOR_OK;
         do {
             bool ok = true;
-            for (int i = 0; i < 7 && ok; i++) ok = dalloc(ds[i], n) == hipSuccess &&
-                hipMemcpyAsync(*ds[i], hs[i], n * sizeof(double), kin, s) == hipSuccess;
-            ok = ok && dalloc(&raw.flv, n) == hipSuccess &&
-                 hipMemcpyAsync(raw.flv, flv, n * sizeof(int), kin, s) == hipSuccess;
+            if (kin == hipMemcpyHostToDevice) {
+                for (int i = 0; i < 7 && ok; i++) ok = dalloc(ds[i], n) == hipSuccess &&
+                    hipMemcpyAsync(*ds[i], hs[i], n * sizeof(double), kin, s) == hipSuccess;
+                ok = ok && dalloc(&raw.flv, n) == hipSuccess &&
+                     hipMemcpyAsync(raw.flv, flv, n * sizeof(int), kin, s) == hipSuccess;
+            } else {   // the caller's device arrays are read where they are
+                for (int i = 0; i < 7; i++) *ds[i] = const_cast<double *>(hs[i]);
+                raw.flv = const_cast<int32_t *>(flv);
+            }
             ok = ok && dalloc(&d_tile, n) == hipSuccess && dalloc(&d_count, ng) == hipSuccess &&
                  dalloc(&d_fill, ng) == hipSuccess && dalloc(&d_off, ng + 1) == hipSuccess;
             ok = ok && hipMemsetAsync(d_count, 0, ng * sizeof(int), s) == hipSuccess &&
                  hipMemsetAsync(d_err, 0, sizeof(int), s) == hipSuccess;
             if (!ok) { rc = fail(PICTOR_ERR_HIP, "adjoint: device allocation or copy failed"); break; }
-            launch_raw_tiles_f64(c->g, c->ph, tp, raw, n, 1, d_tile, d_count, d_err, s);
+            constexpr bool f32 = std::is_same<R, float>::value;
+            const double *const rawp[6] = {raw.x, raw.y, raw.z, raw.u, raw.v, raw.w};
+            launch_raw_tiles_f64(c->g, c->ph, tp, raw, n, f32 ? 1 : 0, d_tile, d_count, d_err, s);
+            if (!f32) launch_fa_range64(ap, rawp, n, d_err, s);
             std::vector<int> cnt(ng);
             int err = 0;
             if (hipGetLastError() != hipSuccess ||
@@ -421,10 +466,24 @@ struct AdjEngine : AdjEngineBase {
                 rc = fail(PICTOR_ERR_HIP, "adjoint: tile count failed");
                 break;
             }
-            if (err) { rc = fail(PICTOR_ERR_ARG, "adjoint: particle outside the physical cells"); break; }
+            if (err) {
+                rc = fail(PICTOR_ERR_ARG, f32 ? "adjoint: particle outside the physical cells"
+                                              : "adjoint: particle outside the physical cells or 2-D z outside [1,2)");
+                break;
+            }
             std::vector<long long> counts(ng);
             for (size_t i = 0; i < ng; i++) counts[i] = cnt[i];
             engine_layout(tp, c->ph.c, counts, cap_factor, h_base, h_cap, lay_total);
+            if (!f32) {
+                // the unsorted engine holds n particles a state instead of a layout's slots
+                const long long states = nseg + std::max(seg, 2);
+                const long long need = lay_total * (states * 56 + 2 * 48 + 4LL * seg) + ncell * (48LL * seg + 72);
+                size_t mfree = 0, mtotal = 0;
+                if (lay_total >= 0x7fffffffLL || hipMemGetInfo(&mfree, &mtotal) != hipSuccess || need > 0.95 * (double)mfree) {
+                    rc = kUseUnsorted;
+                    break;
+                }
+            }
             if (lay_total >= 0x7fffffffLL) { rc = fail(PICTOR_ERR_CAPACITY, "adjoint: tile bins beyond 2^31 slots"); break; }
             if ((rc = setup_bins())) break;
             // centre-bin bases of every group, fill counters, centre counts of checkpoint 0
@@ -443,7 +502,10 @@ struct AdjEngine : AdjEngineBase {
                 rc = fail(PICTOR_ERR_HIP, "adjoint: layout upload failed");
                 break;
             }
-            launch_raw_scatter_split(c->g, c->ph, tp, raw, n, d_tile, d_off, d_fill, d_count, ck2[0], s);
+            if constexpr (std::is_same<R, float>::value)
+                launch_raw_scatter_split(c->g, c->ph, tp, raw, n, d_tile, d_off, d_fill, d_count, ck2[0], s);
+            else
+                launch_fa_load64(ap, rawp, raw.flv, n, d_tile, d_off, d_fill, d_count, ck2[0], s);
             if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
                 rc = fail(PICTOR_ERR_HIP, "adjoint: particle scatter failed");
         } while (false);
@@ -451,33 +513,49 @@ struct AdjEngine : AdjEngineBase {
         return rc;
     }
 
-    // one step of the tile-sorted engine: state (in, cin) -> (out, cout); j >= 0
-    // records step j of a segment (E, B as the push reads them, slot map)
-    int fwd_bins(PartSplit in, const int *cin, PartSplit out, int *cout, int j)
+    // the push of one step of the tile-sorted engine: state (in, cin) -> (out, cout) in the
+    // fields fE, fB; dst (may be null) records the slots
+    void push_bins(R *const *fE, R *const *fB, State in, const int *cin, State out, int *cout, int *dst)
     {
-        hipStream_t s = c->stream;
-        float *const *fE = reinterpret_cast<float *const *>(E);
-        float *const *fB = reinterpret_cast<float *const *>(B);
-        launch_update_b_half<float>(c->g, c->ph, fE, fB, s);
-        launch_ghost_copy<float>(c->g, fB, s);
-        if (j >= 0) {
-            float *dst[6] = {sfE[3 * j], sfE[3 * j + 1], sfE[3 * j + 2], sfB[3 * j], sfB[3 * j + 1], sfB[3 * j + 2]};
-            float *src[6] = {fE[0], fE[1], fE[2], fB[0], fB[1], fB[2]};
-            launch_copy_n<float>(dst, src, 6, ncell, s);
-        }
-        launch_fill_zero_n<double>(J, 3, ncell, s);
         BinsP bins{d_base, d_cap, cin, cout};
         SpillP sp{d_spill, spill_cap, d_err};
-        launch_push2d_split_track(c->tp.T, c->g, c->ph, c->tp, fE, fB, J, in, out, bins, spill, sp,
-                                  j >= 0 ? dstv[j] : nullptr, s);
-        launch_update_b_half<float>(c->g, c->ph, fE, fB, s);
-        launch_ghost_copy<float>(c->g, fB, s);
-        launch_current_fold<double>(c->g, J, s);
-        if (c->curr_filter > 0) launch_smoothen_current(c->g, c->curr_filter, J, Jt, s);
-        launch_update_e_pair(c->g, c->ph, fE, Elo, fB, J, ctx_jscale, true, true, s);
-        launch_ghost_copy<float>(c->g, fE, s, Elo);
-        HIPTRY(hipGetLastError());
-        return PICTOR_OK;
+        if constexpr (std::is_same<R, float>::value)
+            launch_push2d_split_track(c->tp.T, c->g, c->ph, c->tp, fE, fB, J, in, out, bins, spill, sp, dst, c->stream);
+        else
+            launch_fa_push64(c->g, c->tp, ap, fE, fB, J, in, out, bins, sp, dst, c->stream);
+    }
+
+    // ResetCurrent and the first B half step on (fE, fB), in place
+    void first_half(R *const *fE, R *const *fB)
+    {
+        FieldStepP<R> P{};
+        for (int i = 0; i < 3; i++) {
+            P.E[i] = fE[i]; P.B[i] = fB[i]; P.Bn[i] = fB[i]; P.Jz[i] = J[i];
+        }
+        launch_field_b<R>(c->g, c->ph, P, c->stream);
+    }
+
+    // the rest of a step's fields from (fE, fB, Elo, J) into (nE, nB, Elo2), and with `next` the
+    // first half step of the following one; Elo and J swap with their second buffers, J cleared
+    void finish_fields(R *const *fE, R *const *fB, R *const *nE, R *const *nB, bool next)
+    {
+        hipStream_t s = c->stream;
+        if (c->curr_filter > 0) {
+            launch_current_fold<double>(c->g, J, s);
+            launch_smoothen_current(c->g, c->curr_filter, J, Jt, s);
+        }
+        FieldStepP<R> P{};
+        for (int i = 0; i < 3; i++) {
+            P.E[i] = fE[i]; P.B[i] = fB[i]; P.L[i] = Elo[i]; P.J[i] = J[i];
+            P.En[i] = nE[i]; P.Bn[i] = nB[i]; P.Ln[i] = Elo2[i]; P.Jz[i] = J2[i];
+        }
+        P.fold = c->curr_filter > 0 ? 0 : 1;
+        P.next = next ? 1 : 0;
+        launch_field_step<R>(c->g, c->ph, ctx_jscale, P, s);
+        for (int i = 0; i < 3; i++) {
+            std::swap(Elo[i], Elo2[i]);
+            std::swap(J[i], J2[i]);
+        }
     }
 
     // spill / error flags of the steps since the last reset (synchronises)
@@ -573,11 +651,11 @@ struct AdjEngine : AdjEngineBase {
         return PICTOR_OK;
     }
 
-    int restore_ck(int k)
+    int restore_ck(int k, R *const *fE, R *const *fB)
     {
         for (int i = 0; i < 3; i++) {
-            HIPTRY(hipMemcpyAsync(E[i], ckE[3 * k + i], ncell * sizeof(R), hipMemcpyDeviceToDevice, c->stream));
-            HIPTRY(hipMemcpyAsync(B[i], ckB[3 * k + i], ncell * sizeof(R), hipMemcpyDeviceToDevice, c->stream));
+            HIPTRY(hipMemcpyAsync(fE[i], ckE[3 * k + i], ncell * sizeof(R), hipMemcpyDeviceToDevice, c->stream));
+            HIPTRY(hipMemcpyAsync(fB[i], ckB[3 * k + i], ncell * sizeof(R), hipMemcpyDeviceToDevice, c->stream));
             if (Elo[i]) HIPTRY(hipMemcpyAsync(Elo[i], ckElo[3 * k + i], ncell * 4, hipMemcpyDeviceToDevice, c->stream));
         }
         return PICTOR_OK;
@@ -600,18 +678,27 @@ struct AdjEngine : AdjEngineBase {
         HIPTRY(hipEventRecord(ev[0], s));
         if (fast) {
             // the step that ends a segment writes the next checkpoint directly
-            PartSplit a = ck2[0];
+            State a = ck2[0];
             int *ac = ck_cnt[0];
             for (int t = 0; t < nsteps; t++) {
-                if (t % seg == 0 && (rc = save_ck(t / seg))) return rc;
+                if (t % seg == 0) {
+                    if ((rc = save_ck(t / seg))) return rc;
+                    first_half(E, B);
+                }
                 const int k1 = (t + 1) / seg;
-                const bool to_ck = (t + 1) % seg == 0 && k1 < nseg;
-                PartSplit b = to_ck ? ck2[k1] : st2[1 + (t % 2)];
+                const bool ends = (t + 1) % seg == 0, to_ck = ends && k1 < nseg;
+                State b = to_ck ? ck2[k1] : st2[1 + (t % 2)];
                 int *bc = to_ck ? ck_cnt[k1] : cntv[1 + (t % 2)];
-                if ((rc = fwd_bins(a, ac, b, bc, -1))) return rc;
+                push_bins(E, B, a, ac, b, bc, nullptr);
+                finish_fields(E, B, E2, B2, !ends && t + 1 < nsteps);
+                for (int i = 0; i < 3; i++) {
+                    std::swap(E[i], E2[i]);
+                    std::swap(B[i], B2[i]);
+                }
                 a = b;
                 ac = bc;
             }
+            HIPTRY(hipGetLastError());
         } else {
             // ping-pong between st[1] and st[2] (st[1] alone when a segment is one step)
             EPart<R> a = ck[0];
@@ -668,38 +755,44 @@ struct AdjEngine : AdjEngineBase {
         for (int k = nseg - 1; k >= 0; k--) {
             const int t0 = k * seg, t1 = std::min(nsteps, t0 + seg), L = t1 - t0;
             HIPTRY(hipEventRecord(ev[0], s));
-            if ((rc = restore_ck(k))) return rc;
             if (fast) {
+                if ((rc = restore_ck(k, &sfE[0], &sfB[0]))) return rc;
+                first_half(&sfE[0], &sfB[0]);
                 auto S = [&](int j) { return j == 0 ? ck2[k] : st2[j]; };
                 auto C = [&](int j) { return j == 0 ? ck_cnt[k] : cntv[j]; };
-                for (int j = 0; j < L; j++)
-                    if ((rc = fwd_bins(S(j), C(j), st2[j + 1], cntv[j + 1], j))) return rc;
+                for (int j = 0; j < L; j++) {
+                    push_bins(&sfE[3 * j], &sfB[3 * j], S(j), C(j), st2[j + 1], cntv[j + 1], dstv[j]);
+                    // the fields after the segment's last push are in the next checkpoint
+                    if (j + 1 < L)
+                        finish_fields(&sfE[3 * j], &sfB[3 * j], &sfE[3 * (j + 1)], &sfB[3 * (j + 1)], true);
+                }
+                HIPTRY(hipGetLastError());
                 HIPTRY(hipEventRecord(ev[1], s));
                 if ((rc = check_bins(false))) return rc;
                 // adjoint of state L of this segment: zero after the last step, else the
                 // adjoint of the next checkpoint moved to the recomputed slot order
                 if (k == nseg - 1) {
-                    for (float *p : {fa[cur].ox, fa[cur].oy, fa[cur].oz, fa[cur].u, fa[cur].v, fa[cur].w})
-                        launch_fill_zero<float>(p, lay_total, s);
+                    R *const z[6] = {fa[cur].ox, fa[cur].oy, fa[cur].oz, fa[cur].u, fa[cur].v, fa[cur].w};
+                    launch_fill_zero_n<R>(z, 6, lay_total, s);
                 } else {
-                    launch_fa_slots(tp, 0, d_base, ck_cnt[k + 1], ck2[k + 1].id, pos, fa[cur], fa[cur], 1.0, nullptr,
+                    launch_fa_slots<R>(tp, 0, d_base, ck_cnt[k + 1], ck2[k + 1].id, pos, fa[cur], fa[cur], 1.0, nullptr,
                                     nullptr, nullptr, s);
-                    launch_fa_slots(tp, 1, d_base, C(L), S(L).id, pos, fa[cur], fa[1 - cur], 1.0, nullptr, nullptr,
+                    launch_fa_slots<R>(tp, 1, d_base, C(L), S(L).id, pos, fa[cur], fa[1 - cur], 1.0, nullptr, nullptr,
                                     nullptr, s);
                     cur = 1 - cur;
                 }
                 for (int j = L - 1; j >= 0; j--) {
                     const int src = cur;
-                    float *fE[3] = {sfE[3 * j], sfE[3 * j + 1], sfE[3 * j + 2]};
-                    float *fB[3] = {sfB[3 * j], sfB[3 * j + 1], sfB[3 * j + 2]};
+                    R *const *fE = &sfE[3 * j], *const *fB = &sfB[3 * j];
                     rc = rev_step([&]() {
-                        launch_fa_adjoint(c->g, tp, ap, fE, fB, Jadj, d_base, C(j), S(j), dstv[j], fa[src], fa[1 - src],
+                        launch_fa_adjoint<R>(c->g, tp, ap, fE, fB, Jadj, d_base, C(j), S(j), dstv[j], fa[src], fa[1 - src],
                                           gE, gB, s);
                     });
                     if (rc) return rc;
                     cur = 1 - cur;
                 }
             } else {
+                if ((rc = restore_ck(k, E, B))) return rc;
                 // state j of the segment: the checkpoint for j = 0, st[j] after that
                 auto S = [&](int j) { return j == 0 ? ck[k] : st[j]; };
                 for (int j = 0; j < L; j++)
@@ -719,20 +812,24 @@ struct AdjEngine : AdjEngineBase {
             t_adj += m2;
         }
         if (du || dv || dw) {
-            double *d[3] = {};
-            for (int i = 0; i < 3; i++) HIPTRY(dalloc(&d[i], n));
-            if (fast) {
-                for (int i = 0; i < 3; i++) launch_fill_zero<double>(d[i], n, s);
-                launch_fa_slots(tp, 2, d_base, ck_cnt[0], ck2[0].id, pos, fa[cur], fa[cur], scale, d[0], d[1], d[2], s);
+            // straight to the caller's device arrays; a copy for host arrays
+            double *h[3] = {du, dv, dw}, *d[3] = {};
+            const bool direct = kout == hipMemcpyDeviceToDevice;
+            for (int i = 0; i < 3; i++) {
+                if (direct && h[i]) d[i] = h[i];
+                else HIPTRY(dalloc(&d[i], n));
+            }
+            if (fast) {   // every particle has a slot of checkpoint 0
+                launch_fa_slots<R>(tp, 2, d_base, ck_cnt[0], ck2[0].id, pos, fa[cur], fa[cur], scale, d[0], d[1], d[2], s);
             } else {
                 launch_eng_store_grad<R>(adj, scale, d[0], d[1], d[2], n, s);
             }
             HIPTRY(hipGetLastError());
-            double *h[3] = {du, dv, dw};
             for (int i = 0; i < 3; i++)
-                if (h[i]) HIPTRY(hipMemcpyAsync(h[i], d[i], n * sizeof(double), kout, s));
+                if (h[i] && d[i] != h[i]) HIPTRY(hipMemcpyAsync(h[i], d[i], n * sizeof(double), kout, s));
             HIPTRY(hipStreamSynchronize(s));
-            for (int i = 0; i < 3; i++) dfree(d[i]);
+            for (int i = 0; i < 3; i++)
+                if (d[i] != h[i]) dfree(d[i]);
         }
         HIPTRY(hipStreamSynchronize(s));
         return PICTOR_OK;
@@ -773,8 +870,18 @@ int adj_forward(pictor_ctx *c, int64_t n, const double *q, const double *x, cons
         rc = e->setup(c, n, nsteps, segment, engine == 0, cf);
         if (!rc) rc = e->load(q, x, y, z, u, v, w, flv);
         if (!rc) rc = e->forward();
+        if (rc == kUseUnsorted) {
+            engine = 1;
+            repeats = 0;
+            continue;
+        }
         if (rc != kRetryLayout) break;
         if (++repeats > 3) {
+            if (std::is_same<R, double>::value) {
+                engine = 1;
+                repeats = 0;
+                continue;
+            }
             rc = fail(PICTOR_ERR_CAPACITY, "adjoint: tile bins overflowed at 12x the initial tile population");
             break;
         }

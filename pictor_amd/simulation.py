@@ -328,7 +328,7 @@ class Simulation:
         check(lib().pictor_adjoint_release(self._ctx))
 
     def adjoint_engine(self, engine):
-        """'sorted' (tile-sorted FP32 kernels, the default) or 'unsorted'."""
+        """'sorted' (tile-sorted kernels, the default) or 'unsorted'."""
         check(lib().pictor_adjoint_engine(self._ctx, {"sorted": 0, "unsorted": 1}[engine]))
 
 
