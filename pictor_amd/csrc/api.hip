@@ -857,6 +857,7 @@ int pictor_finalize(pictor_ctx *c)
     dfree(c->d_partial); dfree(c->d_rho);
     bc_release(c);
     if (c->h_flags) hipHostFree(c->h_flags);
+    c->ring.release();
     for (int i = 0; i < 23; i++) if (c->ev[i]) hipEventDestroy(c->ev[i]);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
@@ -910,22 +911,18 @@ int pictor_download_fields(pictor_ctx *c, double *ex, double *ey, double *ez, do
     void *src[9] = {c->E[0], c->E[1], c->E[2], c->B[0], c->B[1], c->B[2], c->J[0], c->J[1], c->J[2]};
     const size_t n = (size_t)c->g.ncell;
     const bool f64 = c->form == PICTOR_FORM_FP64 || c->cylm;
-    double *tmp = nullptr;
-    if (!f64) HIPTRY(dalloc(&tmp, n));
+    std::vector<HostItem> items;
     for (int i = 0; i < 9; i++) {
         if (!dst[i]) continue;
-        if (f64) {
-            HIPTRY(hipMemcpyAsync(dst[i], src[i], n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        } else {
-            if (i < 3) launch_pair_to_f64((const float *)src[i], c->Elo[i], tmp, (long long)n, c->stream);
-            else if (i < 6) launch_convert_fields_f64((const float *)src[i], tmp, (long long)n, c->stream);
-            else launch_convert_jfix((const double *)src[i], tmp, (long long)n, jscale(c), c->stream);
-            HIPTRY(hipMemcpyAsync(dst[i], tmp, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-            HIPTRY(hipStreamSynchronize(c->stream));
+        HostItem it = host_raw(dst[i], src[i], n, sizeof(double));
+        if (!f64) {
+            it.kind = i < 3 ? HostItem::kPair : i < 6 ? HostItem::kFloat : HostItem::kScaled;
+            if (i < 3) it.lo = c->Elo[i];
+            it.scale = jscale(c);
         }
+        items.push_back(it);
     }
-    HIPTRY(hipStreamSynchronize(c->stream));
-    if (tmp) dfree(tmp);
+    HIPTRY(deliver(c->ring, items, c->stream));
     return PICTOR_OK;
 }
 
@@ -958,9 +955,9 @@ int pictor_filtered_efield(pictor_ctx *c, int32_t passes, double *fx, double *fy
     launch_smoothen_current(c->g, passes, F, T, c->stream);
     launch_ghost_copy<double>(c->g, F, c->stream);
     double *dst[3] = {fx, fy, fz};
-    for (int i = 0; i < 3; i++)
-        HIPTRY(hipMemcpyAsync(dst[i], F[i], n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    const hipError_t e = hipStreamSynchronize(c->stream);
+    std::vector<HostItem> items;
+    for (int i = 0; i < 3; i++) items.push_back(host_raw(dst[i], F[i], n, sizeof(double)));
+    const hipError_t e = deliver(c->ring, items, c->stream);
     release();
     if (e != hipSuccess) return fail(PICTOR_ERR_HIP, std::string("filtered E: ") + hipGetErrorString(e));
     return PICTOR_OK;
@@ -1129,12 +1126,15 @@ static int download_particles_impl(pictor_ctx *c, int64_t cap, double *q, double
     HIPTRY(hipGetLastError());
     double *hd[7] = {q, x, y, z, u, v, w};
     double *dd[7] = {st.q, st.x, st.y, st.z, st.u, st.v, st.w};
-    for (int i = 0; i < 7; i++)
-        if (hd[i]) HIPTRY(hipMemcpyAsync(hd[i], dd[i], n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    if (flv) HIPTRY(hipMemcpyAsync(flv, st.flv, n * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    if (tile) HIPTRY(hipMemcpyAsync(tile, d_tile, n * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    if (tag) HIPTRY(hipMemcpyAsync(tag, st.tag, n * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    HIPTRY(hipStreamSynchronize(c->stream));
+    std::vector<HostItem> items;
+    auto put = [&](void *dst, const void *src, size_t elem) {
+        if (dst) items.push_back(host_raw(dst, src, (size_t)n, elem));
+    };
+    for (int i = 0; i < 7; i++) put(hd[i], dd[i], sizeof(double));
+    put(flv, st.flv, sizeof(int));
+    put(tile, d_tile, sizeof(int));
+    put(tag, st.tag, sizeof(int32_t));
+    HIPTRY(deliver(c->ring, items, c->stream));
     dfree(d_off); dfree(d_tile);
     free_f64(st); free_split(ss);
     return PICTOR_OK;

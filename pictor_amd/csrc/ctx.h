@@ -8,6 +8,7 @@
 #include "pictor_common.h"
 #include "cyl.h"
 #include "cylm.h"
+#include "hostcopy.h"
 
 struct pictor_ctx;
 
@@ -84,6 +85,7 @@ struct pictor_ctx {
     void *J[3] = {nullptr, nullptr, nullptr};
     // split form: the low FP32 part of E (E = hi + lo, hi in E[]), see launch_update_e_pair
     float *Elo[3] = {nullptr, nullptr, nullptr};
+    pictor::HostRing ring;   // downloads
     // second buffers of E, B, Elo and J: a fused step reads one set and writes the other
     void *E2[3] = {nullptr, nullptr, nullptr}, *B2[3] = {nullptr, nullptr, nullptr}, *J2[3] = {nullptr, nullptr, nullptr};
     float *Elo2[3] = {nullptr, nullptr, nullptr};

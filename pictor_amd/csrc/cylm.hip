@@ -1605,9 +1605,11 @@ int cylm_download_particles(pictor_ctx *c, long long cap, double *q, double *x, 
         const PartF64 &p = c->pcyl;
         double *hd[7] = {q, x, y, z, u, v, w};
         double *dd[7] = {p.q, p.x, p.y, p.z, p.u, p.v, p.w};
+        std::vector<HostItem> items;
         for (int i = 0; i < 7; i++)
-            if (hd[i]) HIPTRY(hipMemcpy(hd[i], dd[i], n * sizeof(double), hipMemcpyDeviceToHost));
-        if (flv) HIPTRY(hipMemcpy(flv, p.flv, n * sizeof(int), hipMemcpyDeviceToHost));
+            if (hd[i]) items.push_back(host_raw(hd[i], dd[i], (size_t)n, sizeof(double)));
+        if (flv) items.push_back(host_raw(flv, p.flv, (size_t)n, sizeof(int)));
+        HIPTRY(deliver(c->ring, items, c->stream));
         return PICTOR_OK;
     }
     // the split record in the FP64 layout: x = i + ox, z = k + oz (exact), theta = turns * 2 pi / 2^32

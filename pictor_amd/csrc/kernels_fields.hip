@@ -445,16 +445,6 @@ __global__ void k_cvt_f32(const double *s, float *d, long long n)
     long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n) d[t] = (float)s[t];
 }
-__global__ void k_cvt_f64(const float *s, double *d, long long n)
-{
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) d[t] = (double)s[t];
-}
-__global__ void k_cvt_jfix(const double *s, double *d, long long n, double scale)
-{
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) d[t] = (double)s[t] * scale;
-}
 
 inline unsigned nblocks(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
@@ -620,14 +610,6 @@ void launch_pair_to_f64(const float *hi, const float *lo, double *dst, long long
 void launch_convert_fields_f32(const double *src, float *dst, long long n, hipStream_t s)
 {
     hipLaunchKernelGGL(k_cvt_f32, dim3(nblocks(n, 256)), dim3(256), 0, s, src, dst, n);
-}
-void launch_convert_fields_f64(const float *src, double *dst, long long n, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_cvt_f64, dim3(nblocks(n, 256)), dim3(256), 0, s, src, dst, n);
-}
-void launch_convert_jfix(const double *src, double *dst, long long n, double scale, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_cvt_jfix, dim3(nblocks(n, 256)), dim3(256), 0, s, src, dst, n, scale);
 }
 
 template void launch_update_b_half<double>(const GridP &, const PhysP &, double *const[3], double *const[3], hipStream_t);

@@ -207,8 +207,6 @@ void launch_update_e_pair(const GridP &g, const PhysP &ph, float *const E[3], fl
 void launch_pair_from_f64(const double *src, float *hi, float *lo, long long n, hipStream_t s);
 void launch_pair_to_f64(const float *hi, const float *lo, double *dst, long long n, hipStream_t s);
 void launch_convert_fields_f32(const double *src, float *dst, long long n, hipStream_t s);
-void launch_convert_fields_f64(const float *src, double *dst, long long n, hipStream_t s);
-void launch_convert_jfix(const double *src, double *dst, long long n, double scale, hipStream_t s);
 
 // ---------------- launchers (kernels_push.hip) ----------------
 struct BinsP {

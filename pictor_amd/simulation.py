@@ -110,7 +110,7 @@ class Simulation:
         check(lib().pictor_upload_fields(self._ctx, *[_p(a) for a in arrs]))
 
     def download_fields(self):
-        out = {n: np.zeros(self.shape, order="F") for n in ("Ex", "Ey", "Ez", "Bx", "By", "Bz", "Jx", "Jy", "Jz")}
+        out = {n: np.empty(self.shape, order="F") for n in ("Ex", "Ey", "Ez", "Bx", "By", "Bz", "Jx", "Jy", "Jz")}
         check(lib().pictor_download_fields(self._ctx, *[_p(out[n]) for n in ("Ex", "Ey", "Ez", "Bx", "By", "Bz",
                                                                               "Jx", "Jy", "Jz")]))
         return out
@@ -137,7 +137,7 @@ class Simulation:
     def filtered_efield(self, passes):
         """SetFilteredEfldGPU (fields_gpu.F90:70-90): E after `passes` rounds of the 1-2-1
         filter and the halo copy (the field the reference's test particles feel)."""
-        out = {n: np.zeros(self.shape, order="F") for n in ("Ex", "Ey", "Ez")}
+        out = {n: np.empty(self.shape, order="F") for n in ("Ex", "Ey", "Ez")}
         check(lib().pictor_filtered_efield(self._ctx, passes, *[_p(out[n]) for n in ("Ex", "Ey", "Ez")]))
         return out
 
