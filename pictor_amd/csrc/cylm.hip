@@ -341,91 +341,212 @@ struct DepMove {
     double pa[3], pt[3];
 };
 
+// Every contribution is a product a b; add(component, slot, half, di, dk, a, b) receives it for the
+// node (i1 + di, k1 + dk) (half 0) or (i2 + di, k2 + dk) (half 1).
 template <class Add>
 __device__ inline void modal_deposit(const DepMove &d, Add add)
 {
+    const double Vx1 = 1.0 - d.Wx1, Vz1 = 1.0 - d.Wz1, Vx2 = 1.0 - d.Wx2, Vz2 = 1.0 - d.Wz2;
 #pragma unroll
     for (int s = 0; s < 3; s++) {
-        add(0, s, d.i1, d.k1, d.pa[s] * d.Fx1 * (1.0 - d.Wz1));
-        add(0, s, d.i1, d.k1 + 1, d.pa[s] * d.Fx1 * d.Wz1);
-        add(2, s, d.i1, d.k1, d.pa[s] * d.Fz1 * (1.0 - d.Wx1));
-        add(2, s, d.i1 + 1, d.k1, d.pa[s] * d.Fz1 * d.Wx1);
-        add(0, s, d.i2, d.k2, d.pa[s] * d.Fx2 * (1.0 - d.Wz2));
-        add(0, s, d.i2, d.k2 + 1, d.pa[s] * d.Fx2 * d.Wz2);
-        add(2, s, d.i2, d.k2, d.pa[s] * d.Fz2 * (1.0 - d.Wx2));
-        add(2, s, d.i2 + 1, d.k2, d.pa[s] * d.Fz2 * d.Wx2);
+        const double fx1 = d.pa[s] * d.Fx1, fz1 = d.pa[s] * d.Fz1, fx2 = d.pa[s] * d.Fx2, fz2 = d.pa[s] * d.Fz2;
+        add(0, s, 0, 0, 0, fx1, Vz1);
+        add(0, s, 0, 0, 1, fx1, d.Wz1);
+        add(2, s, 0, 0, 0, fz1, Vx1);
+        add(2, s, 0, 1, 0, fz1, d.Wx1);
+        add(0, s, 1, 0, 0, fx2, Vz2);
+        add(0, s, 1, 0, 1, fx2, d.Wz2);
+        add(2, s, 1, 0, 0, fz2, Vx2);
+        add(2, s, 1, 1, 0, fz2, d.Wx2);
     }
+    const double vx = 1.0 - d.wx, vz = 1.0 - d.wz;
 #pragma unroll
     for (int s = 0; s < 3; s++) {
-        add(1, s, d.i2, d.k2, d.pt[s] * (1.0 - d.wx) * (1.0 - d.wz));
-        add(1, s, d.i2 + 1, d.k2, d.pt[s] * d.wx * (1.0 - d.wz));
-        add(1, s, d.i2, d.k2 + 1, d.pt[s] * (1.0 - d.wx) * d.wz);
-        add(1, s, d.i2 + 1, d.k2 + 1, d.pt[s] * d.wx * d.wz);
+        const double tl = d.pt[s] * vx, tr = d.pt[s] * d.wx;
+        add(1, s, 1, 0, 0, tl, vz);
+        add(1, s, 1, 1, 0, tr, vz);
+        add(1, s, 1, 0, 1, tl, d.wz);
+        add(1, s, 1, 1, 1, tr, d.wz);
     }
 }
 
+// modal_deposit for a particle that stays in its cell (i1 = i2, k1 = k2): both r-z
+// half-segments land on the same nodes; add(component, slot, di, dk, value) gets their sum,
+// term(a1, b1, a2, b2)
+template <class Term, class Add>
+__device__ inline void modal_deposit_same_cell(const DepMove &d, Term term, Add add)
+{
+    const double Vx1 = 1.0 - d.Wx1, Vz1 = 1.0 - d.Wz1, Vx2 = 1.0 - d.Wx2, Vz2 = 1.0 - d.Wz2;
+#pragma unroll
+    for (int s = 0; s < 3; s++) {
+        const double fx1 = d.pa[s] * d.Fx1, fz1 = d.pa[s] * d.Fz1, fx2 = d.pa[s] * d.Fx2, fz2 = d.pa[s] * d.Fz2;
+        add(0, s, 0, 0, term(fx1, Vz1, fx2, Vz2));
+        add(0, s, 0, 1, term(fx1, d.Wz1, fx2, d.Wz2));
+        add(2, s, 0, 0, term(fz1, Vx1, fz2, Vx2));
+        add(2, s, 1, 0, term(fz1, d.Wx1, fz2, d.Wx2));
+    }
+    const double vx = 1.0 - d.wx, vz = 1.0 - d.wz;
+#pragma unroll
+    for (int s = 0; s < 3; s++) {
+        const double tl = d.pt[s] * vx, tr = d.pt[s] * d.wx;
+        add(1, s, 0, 0, term(tl, vz));
+        add(1, s, 1, 0, term(tr, vz));
+        add(1, s, 0, 1, term(tl, d.wz));
+        add(1, s, 1, 1, term(tr, d.wz));
+    }
+}
+
+// a value the compiler takes to change here: without it the products of modal_deposit are hoisted
+// out of the loop over the windows and hold 30 registers more through it (3 waves per SIMD, not 4)
+__device__ inline void pin(double &x) { asm volatile("" : "+v"(x)); }
+__device__ inline void pin(DepMove &d)
+{
+    pin(d.Fx1); pin(d.Fz1); pin(d.Fx2); pin(d.Fz2);
+    pin(d.Wx1); pin(d.Wz1); pin(d.Wx2); pin(d.Wz2);
+    pin(d.wx); pin(d.wz); pin(d.pt[0]); pin(d.pt[1]); pin(d.pt[2]);
+}
+
+// a contribution in FP64
+struct Product {
+    __device__ double operator()(double a, double b) const { return a * b; }
+    __device__ double operator()(double a1, double b1, double a2, double b2) const { return a1 * b1 + a2 * b2; }
+};
+
+// minimum over the wave, in every lane: row shifts and broadcasts (DPP), no LDS traffic
 __device__ inline int wave_min(int v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-    return v;
+    const int id = INT_MAX;
+    v = min(v, __builtin_amdgcn_update_dpp(id, v, 0x111, 0xf, 0xf, false));   // row_shr:1
+    v = min(v, __builtin_amdgcn_update_dpp(id, v, 0x112, 0xf, 0xf, false));   // row_shr:2
+    v = min(v, __builtin_amdgcn_update_dpp(id, v, 0x114, 0xf, 0xf, false));   // row_shr:4
+    v = min(v, __builtin_amdgcn_update_dpp(id, v, 0x118, 0xf, 0xf, false));   // row_shr:8
+    v = min(v, __builtin_amdgcn_update_dpp(id, v, 0x142, 0xa, 0xf, false));   // row_bcast:15, rows 1 and 3
+    v = min(v, __builtin_amdgcn_update_dpp(id, v, 0x143, 0xc, 0xf, false));   // row_bcast:31, rows 2 and 3
+    return __builtin_amdgcn_readlane(v, 63);
 }
-__device__ inline int wave_max(int v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-    return v;
-}
+// ~v reverses the order of the integers
+__device__ inline int wave_max(int v) { return ~wave_min(~v); }
 
 // mode cells of the block's deposit window held in LDS: 9 accumulators (3 components x
-// 3 slots) per (i, k) cell, FP64.  A window of at most kDepCells / 4 cells keeps 4
-// interleaved copies of each accumulator (lane l adds into copy l % 4): the particles of
-// one cell sit in adjacent lanes and would otherwise serialise on the same LDS words
+// 3 slots) per (i, k) cell, FP64 or 64-bit counts.  A window of at most kDepCells / R cells keeps
+// R = 2, 4 or kDepCopies copies of its accumulators (lane l adds into copy l % R): the particles of
+// one cell sit in adjacent lanes and would otherwise serialise on the same LDS words.
+// Copy r of a cell is slot L = cell R + r; its accumulator cs = 3 component + slot is word
+// 36 (L / 4) + 4 cs + L % 4: the nine of a node are immediate offsets of one address (an address
+// each cost the split push a quarter of its time in 32-bit multiplies), and the copies of 8 (R = 4)
+// neighbouring cells cover the 64 banks once.
 constexpr int kDepCells = 448;
-constexpr int kDepCopies = 4;
-// when the block's particles spread wider than kDepCells cells (electrons expelled,
-// crossing the axis or trapped in the wake, far from their array neighbours), the window
-// is a box of kBoxI x kBoxK cells around the block's first depositing particle; the
-// particles outside it add to J directly
+constexpr int kDepCopies = 8;
+constexpr int kDepWords = 9 * kDepCells;
+// words of the nodes (di, dk) of a cell: w[di + 2 dk]
+struct Corners {
+    int w[4];
+};
+struct DepWin {
+    int bil, bkl, wi, wk;   // i in [bil, bil + wi), k in [bkl, bkl + wk)
+    int R;                  // copies
+    bool box;               // some particles may lie outside
+    __device__ static int word(int L) { return 36 * (L >> 2) + (L & 3); }
+    // the word of accumulator 0 of lane copy rl of node (i, k)
+    __device__ int at(int i, int k, int rl) const { return word(((k - bkl) * wi + (i - bil)) * R + rl); }
+    __device__ Corners corners(int i, int k, int rl) const
+    {
+        return Corners{{at(i, k, rl), at(i + 1, k, rl), at(i, k + 1, rl), at(i + 1, k + 1, rl)}};
+    }
+    __device__ bool holds(const DepMove &d) const
+    {
+        return min(d.i1, d.i2) >= bil && max(d.i1, d.i2) + 1 < bil + wi && min(d.k1, d.k2) >= bkl &&
+               max(d.k1, d.k2) + 1 < bkl + wk;
+    }
+};
+// when the block's particles spread wider than kDepCells cells (a block whose sorted particles run
+// over the end of a row of cells and into the next; electrons expelled, crossing the axis or trapped
+// in the wake, far from their array neighbours), the window is a box of kBoxI x kBoxK cells around the
+// block's first depositing particle, and those outside it go through another window, up to kDepPasses.
+// The last kDepFew or fewer add to J directly: a row of cells is 30 blocks at 480 x 16 particles, and
+// with everything outside the first box added directly the block over its end made the push 20 %
+// slower.
+constexpr int kDepPasses = 4, kDepFew = 16;
 constexpr int kBoxI = 28, kBoxK = 4;
 
-// the block's deposit window [bil, bil + wi) x [bkl, bkl + wk); uniform over the block
-__device__ inline void deposit_window(bool dep, const DepMove &d, int (*sred)[4], int *sbox, int &bil, int &bkl,
-                                      int &wi, int &wk, bool &any)
+// the block's deposit window; uniform over the block; false: no particle deposits
+__device__ inline bool deposit_window(bool dep, const DepMove &d, int (*sred)[4], int *sbox, DepWin &W)
 {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int ilo = wave_min(dep ? min(d.i1, d.i2) : INT_MAX), ihi = wave_max(dep ? max(d.i1, d.i2) : INT_MIN);
     const int klo = wave_min(dep ? min(d.k1, d.k2) : INT_MAX), khi = wave_max(dep ? max(d.k1, d.k2) : INT_MIN);
-    const int first = wave_min(dep ? (int)threadIdx.x : INT_MAX);
+    const unsigned long long dm = __ballot(dep);
+    const int first = dm ? (int)(threadIdx.x & ~63u) + __ffsll(dm) - 1 : INT_MAX;
     if (lane == 0) { sred[wv][0] = ilo; sred[wv][1] = ihi; sred[wv][2] = klo; sred[wv][3] = khi; sbox[wv] = first; }
     __syncthreads();
-    int bih = INT_MIN, bkh = INT_MIN, f = INT_MAX;
-    bil = INT_MAX; bkl = INT_MAX;
+    int bil = INT_MAX, bkl = INT_MAX, bih = INT_MIN, bkh = INT_MIN, f = INT_MAX;
 #pragma unroll
     for (int w = 0; w < 4; w++) {
         bil = min(bil, sred[w][0]); bih = max(bih, sred[w][1]);
         bkl = min(bkl, sred[w][2]); bkh = max(bkh, sred[w][3]);
         f = min(f, sbox[w]);
     }
-    any = bil <= bih;
-    if (!any) return;
-    wi = bih + 2 - bil;
-    wk = bkh + 2 - bkl;
-    if ((long long)wi * wk <= kDepCells) return;
-    __syncthreads();   // every thread has read sbox
-    if ((int)threadIdx.x == f) { sbox[0] = min(d.i1, d.i2); sbox[1] = min(d.k1, d.k2); }
-    __syncthreads();
-    bil = sbox[0] - 4;
-    bkl = sbox[1] - 1;
-    wi = kBoxI;
-    wk = kBoxK;
+    if (bil > bih) return false;
+    W.box = false;
+    W.wi = bih + 2 - bil;
+    W.wk = bkh + 2 - bkl;
+    if ((long long)W.wi * W.wk > kDepCells) {
+        __syncthreads();   // every thread has read sbox
+        if ((int)threadIdx.x == f) { sbox[0] = min(d.i1, d.i2); sbox[1] = min(d.k1, d.k2); }
+        __syncthreads();
+        bil = sbox[0] - 4;
+        bkl = sbox[1] - 1;
+        W.box = true;
+        W.wi = kBoxI;
+        W.wk = kBoxK;
+    }
+    // uniform over the block: in scalar registers
+    W.bil = __builtin_amdgcn_readfirstlane(bil);
+    W.bkl = __builtin_amdgcn_readfirstlane(bkl);
+    W.wi = __builtin_amdgcn_readfirstlane(W.wi);
+    W.wk = __builtin_amdgcn_readfirstlane(W.wk);
+    const int cells = W.wi * W.wk;
+    W.R = kDepCopies;                           // cells R <= kDepCells
+    while (W.R > 1 && cells * W.R > kDepCells) W.R >>= 1;
+    return true;
+}
+
+// clears the window's accumulators (8-byte words, sJ on a 16-byte boundary); the barrier is the caller's
+__device__ inline void clear_window(const DepWin &W, void *sJ)
+{
+    const int n = (W.wi * W.wk * W.R + 3) / 4 * 18;
+    for (int e = threadIdx.x; e < n; e += 256) ((ulonglong2 *)sJ)[e] = make_ulonglong2(0ull, 0ull);
+}
+
+// one global add per accumulator that is not zero; value(sum) is what J receives.  i fastest: the
+// adds of a row are neighbours.  The divisions by
+// reciprocals are exact (e + 1/2 below 2^12, at least 1/2 of 1 / wi from the next integer).
+template <class T, class Value>
+__device__ inline void flush_window(const GridP &g, const DepWin &W, const T *sJ, double *const J[3], Value value)
+{
+    const int n = 9 * W.wi * W.wk;
+    const float ri = __builtin_amdgcn_rcpf((float)W.wi), rk = __builtin_amdgcn_rcpf((float)W.wk);
+    for (int e = threadIdx.x; e < n; e += 256) {
+        const int r = (int)(((float)e + 0.5f) * ri), i = e - r * W.wi;
+        const int cs = (int)(((float)r + 0.5f) * rk), k = r - cs * W.wk;
+        const T *a = sJ + DepWin::word((k * W.wi + i) * W.R) + 4 * cs;
+        T v = a[0];
+        if (W.R > 1) v += a[1];
+        if (W.R > 2) v += a[2] + a[3];
+        if (W.R > 4) v += a[36] + a[37] + a[38] + a[39];
+        if (v == 0) continue;
+        const int cc = (cs * 11) >> 5;          // cs / 3
+        unsafeAtomicAdd(&J[cc][mi(g, W.bil + i, cs - 3 * cc, W.bkl + k)], value(v));
+    }
 }
 
 // MoveDepositPrtl: gather, Boris, the local-frame move and rotation (cyl_movdep.F90:14-289),
 // then the modal deposit.  The particles keep the loader's cell order, so the 256 of a
 // block deposit into a small (i, k) window: it is accumulated in LDS and added to J once
-// per cell and accumulator; a block whose window exceeds kDepCells cells adds every
-// contribution to J directly.
+// per cell and accumulator.  Bound by FP64 and address arithmetic (VALU) with 4 waves per SIMD:
+// 1.57 million particles, 1024 x 128 cells, 170 -> 133 us with one address per node, the DPP
+// reductions, a single path per wave and, for a particle that stays in its cell, 28 LDS adds
+// instead of 36.
 __global__ __launch_bounds__(256) void k_cylm_push(GridP g, CylmP q, const double *__restrict__ Ex,
                                                    const double *__restrict__ Ey, const double *__restrict__ Ez,
                                                    const double *__restrict__ Bx, const double *__restrict__ By,
@@ -433,7 +554,7 @@ __global__ __launch_bounds__(256) void k_cylm_push(GridP g, CylmP q, const doubl
                                                    double *__restrict__ Jy, double *__restrict__ Jz, PartF64 P,
                                                    long long n, int *__restrict__ err)
 {
-    __shared__ double sJ[9 * kDepCells];
+    __shared__ __attribute__((aligned(16))) double sJ[kDepWords];
     __shared__ int sred[4][4], sbox[4];
     const long long m = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int flv = m < n ? P.flv[m] : 0;
@@ -503,36 +624,41 @@ __global__ __launch_bounds__(256) void k_cylm_push(GridP g, CylmP q, const doubl
         P.x[m] = x1; P.y[m] = tn; P.z[m] = zn;
         P.u[m] = un; P.v[m] = vn; P.w[m] = wn;
     }
-    // the block's window: i in [bil, bil + wi), k in [bkl, bkl + wk)
-    const int lane = threadIdx.x & 63;
-    int bil, bkl, wi, wk;
-    bool any;
-    deposit_window(dep, d, sred, sbox, bil, bkl, wi, wk, any);
-    if (!any) return;                           // nothing to deposit in this block (uniform)
+    const bool same = d.i1 == d.i2 && d.k1 == d.k2;
     double *J[3] = {Jx, Jy, Jz};
-    const bool inside = dep && min(d.i1, d.i2) >= bil && max(d.i1, d.i2) + 1 < bil + wi && min(d.k1, d.k2) >= bkl &&
-                        max(d.k1, d.k2) + 1 < bkl + wk;
-    if (dep && !inside)
-        modal_deposit(d, [&](int cc, int s, int i, int k, double v) { unsafeAtomicAdd(&J[cc][mi(g, i, s, k)], v); });
-    const int cells = wi * wk;
-    int R = kDepCopies;                         // copies per accumulator: cells * R <= kDepCells
-    while (R > 1 && cells * R > kDepCells) R >>= 1;
-    const int rl = lane & (R - 1);
-    for (int e = threadIdx.x; e < 9 * cells * R; e += 256) sJ[e] = 0.0;
-    __syncthreads();
-    if (inside)
-        modal_deposit(d, [&](int cc, int s, int i, int k, double v) {
-            atomicAdd(&sJ[((cc * 3 + s) * cells + (k - bkl) * wi + (i - bil)) * R + rl], v);
-        });
-    __syncthreads();
-    for (int e = threadIdx.x; e < 9 * cells; e += 256) {
-        double v = 0.0;
-        for (int r = 0; r < R; r++) v += sJ[e * R + r];
-        if (v == 0.0) continue;
-        const int cs = e / cells, cell = e - cs * cells;
-        const int i = bil + cell % wi, k = bkl + cell / wi;
-        unsafeAtomicAdd(&J[cs / 3][mi(g, i, cs % 3, k)], v);
+    bool todo = dep;
+    for (int pass = 0;; pass++) {
+        DepWin W;
+        pin(d);
+        if (!deposit_window(todo, d, sred, sbox, W)) return;   // nothing (left) to deposit: uniform
+        const bool inside = todo && W.holds(d);
+        clear_window(W, sJ);
+        __syncthreads();
+        const int rl = threadIdx.x & (W.R - 1);
+        if (__all(!inside || same)) {   // the same for the whole wave: one path, not both
+            if (inside) {
+                const Corners n2 = W.corners(d.i2, d.k2, rl);
+                modal_deposit_same_cell(d, Product(),
+                                        [&](int cc, int s, int di, int dk, double v) {
+                                            atomicAdd(sJ + n2.w[di + 2 * dk] + 4 * (3 * cc + s), v);
+                                        });
+            }
+        } else if (inside) {
+            const Corners n1 = W.corners(d.i1, d.k1, rl), n2 = W.corners(d.i2, d.k2, rl);
+            modal_deposit(d, [&](int cc, int s, int h, int di, int dk, double a, double b) {
+                atomicAdd(sJ + (h ? n2 : n1).w[di + 2 * dk] + 4 * (3 * cc + s), a * b);
+            });
+        }
+        __syncthreads();
+        flush_window(g, W, sJ, J, [](double v) { return v; });
+        if (!W.box) return;
+        todo = todo && !inside;
+        if (__syncthreads_count(todo) <= kDepFew || pass == kDepPasses - 1) break;
     }
+    if (todo)
+        modal_deposit(d, [&](int cc, int s, int h, int di, int dk, double a, double b) {
+            unsafeAtomicAdd(&J[cc][mi(g, (h ? d.i2 : d.i1) + di, s, (h ? d.k2 : d.k1) + dk)], a * b);
+        });
 }
 
 // The node-centred FP32 copy of E and B that the split push gathers from, rebuilt before
@@ -599,30 +725,26 @@ __device__ inline void gather_nodes(const GridP &g, const float4 *__restrict__ n
 #pragma unroll
     for (int s = 0; s < 3; s++)
 #pragma unroll
-        for (int c = 0; c < 3; c++) { pe[c] += ph[s] * se[6 * s + c]; pb[c] += ph[s] * se[6 * s + 3 + c]; }
+        for (int c = 0; c < 3; c++) {
+            pe[c] += ph[s] * se[6 * s + c];
+            pb[c] += ph[s] * se[6 * s + 3 + c];
+        }
 }
 
-// modal_deposit for a particle that stays in its cell (i1 = i2, k1 = k2): the two
-// r-z half-segments land on the same nodes, so their fixed-point counts are added
-// first (integers below 2^53: exact) and each node takes one add instead of two
-template <class Count, class Add>
-__device__ inline void modal_deposit_same_cell(const DepMove &d, Count count, Add add)
-{
-#pragma unroll
-    for (int s = 0; s < 3; s++) {
-        add(0, s, d.i1, d.k1, count(d.pa[s] * d.Fx1 * (1.0 - d.Wz1)) + count(d.pa[s] * d.Fx2 * (1.0 - d.Wz2)));
-        add(0, s, d.i1, d.k1 + 1, count(d.pa[s] * d.Fx1 * d.Wz1) + count(d.pa[s] * d.Fx2 * d.Wz2));
-        add(2, s, d.i1, d.k1, count(d.pa[s] * d.Fz1 * (1.0 - d.Wx1)) + count(d.pa[s] * d.Fz2 * (1.0 - d.Wx2)));
-        add(2, s, d.i1 + 1, d.k1, count(d.pa[s] * d.Fz1 * d.Wx1) + count(d.pa[s] * d.Fz2 * d.Wx2));
+// the count rint(a b) (a in counts) as a 64-bit integer: |a b| <= 64 kJq = 2^42, and adding
+// 1.5 2^52 rounds it to an integer in the low mantissa bits (ties to even, as rint)
+struct Count {
+    __device__ static double bias() { return 6755399441055744.0; }
+    __device__ long long operator()(double a, double b) const
+    {
+        return __double_as_longlong(__builtin_fma(a, b, bias())) - 0x4338000000000000LL;
     }
-#pragma unroll
-    for (int s = 0; s < 3; s++) {
-        add(1, s, d.i2, d.k2, count(d.pt[s] * (1.0 - d.wx) * (1.0 - d.wz)));
-        add(1, s, d.i2 + 1, d.k2, count(d.pt[s] * d.wx * (1.0 - d.wz)));
-        add(1, s, d.i2, d.k2 + 1, count(d.pt[s] * (1.0 - d.wx) * d.wz));
-        add(1, s, d.i2 + 1, d.k2 + 1, count(d.pt[s] * d.wx * d.wz));
+    __device__ long long operator()(double a1, double b1, double a2, double b2) const
+    {
+        return __double_as_longlong(__builtin_fma(a1, b1, bias())) +
+               (__double_as_longlong(__builtin_fma(a2, b2, bias())) - (long long)0x8670000000000000ULL);
     }
-}
+};
 
 // MoveDepositPrtl of the split form: the push in FP32 on (cell, offset) positions, theta
 // in 2^-32 turns; the deposit in FP64 from the stored old and new positions (exact in
@@ -630,12 +752,16 @@ __device__ inline void modal_deposit_same_cell(const DepMove &d, Count count, Ad
 // count in the LDS window: every sum is exact, so J does not depend on the order of the atomics.
 // Flags: 1 = a particle reached the wall, 2 = a contribution above 64 charge cells (the
 // fixed-point range).
+// Bound by the VALU (75 % of its issue slots, 830 instructions a wave).  31.5 million particles,
+// 4096 x 512 cells, with the node copy: 1451 -> 1077 us.  The range check on the factors, not on
+// each of 44 contributions, one FMA per count, immediate LDS offsets and further windows for a block
+// over the end of a row gave it; 8 accumulator copies; 4 take 2 % longer.
 __global__ __launch_bounds__(256) void k_cylm_push_split(GridP g, CylmP q, const float4 *__restrict__ nf4,
                                                          const float2 *__restrict__ nf2, double *__restrict__ Jx,
                                                          double *__restrict__ Jy, double *__restrict__ Jz, PartCylS P,
                                                          long long n, int *__restrict__ err)
 {
-    __shared__ unsigned long long sJ[9 * kDepCells];
+    __shared__ __attribute__((aligned(16))) long long sJ[kDepWords];
     __shared__ int sred[4][4], sbox[4];
     const long long m = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t cw = m < n ? P.cell[m] : 0u;
@@ -692,7 +818,7 @@ __global__ __launch_bounds__(256) void k_cylm_push_split(GridP g, CylmP q, const
             atomicOr(err, 1);
         } else {
             dep = true;
-            const double qthis = (double)P.q[m] * q.qi;
+            const double qthis = (double)P.q[m] * q.qi * kJq;   // in counts: kJq is a power of two
             const double x0 = i0 + (double)ox, z0 = k0 + (double)oz;
             const double x1 = i2 + (double)ox2, z1 = k2 + (double)oz2;
             d.i1 = i0; d.i2 = i2; d.k1 = k0; d.k2 = k2;
@@ -719,50 +845,54 @@ __global__ __launch_bounds__(256) void k_cylm_push_split(GridP g, CylmP q, const
         P.ox[m] = ox2; P.oz[m] = oz2; P.th[m] = t1;
         P.u[m] = un; P.v[m] = vn; P.w[m] = wn;
     }
-    const int lane = threadIdx.x & 63;
-    int bil, bkl, wi, wk;
-    bool any;
-    deposit_window(dep, d, sred, sbox, bil, bkl, wi, wk, any);
-    if (!any) return;
+    // |a b| <= 64 kJq holds for every contribution if it does for the factors and the weights lie in
+    // [0, 1], as they do for moves of at most one cell; else each contribution is looked at
+    if (dep) {
+        const double L = 64.0 * kJq;
+        const bool fits = fabs(d.Fx1) <= L && fabs(d.Fz1) <= L && fabs(d.Fx2) <= L && fabs(d.Fz2) <= L &&
+                          fabs(d.pt[0]) <= L && fabs(d.pt[1]) <= L && fabs(d.pt[2]) <= L && abs(d.i2 - d.i1) <= 1 &&
+                          abs(d.k2 - d.k1) <= 1;
+        if (!fits) {
+            bool big = false;
+            modal_deposit(d, [&](int, int, int, int, int, double a, double b) { big = big || !(fabs(a * b) <= L); });
+            if (big) atomicOr(err, 2);
+        }
+    }
+    const bool same = d.i1 == d.i2 && d.k1 == d.k2;
+    auto put = [&](int w, long long v) { atomicAdd((unsigned long long *)(sJ + w), (unsigned long long)v); };
     double *J[3] = {Jx, Jy, Jz};
-    bool big = false;
-    // the count rint(v 2^36) as a 64-bit integer: |v| <= 64 keeps v 2^36 below 2^51, where
-    // adding 1.5 2^52 rounds it to an integer in the low mantissa bits (ties to even, as rint)
-    auto count = [&](double v) -> long long {
-        big = big || !(fabs(v) <= 64.0);
-        return __double_as_longlong(v * kJq + 6755399441055744.0) - 0x4338000000000000LL;
-    };
-    const bool inside = dep && min(d.i1, d.i2) >= bil && max(d.i1, d.i2) + 1 < bil + wi && min(d.k1, d.k2) >= bkl &&
-                        max(d.k1, d.k2) + 1 < bkl + wk;
-    if (dep && !inside)
-        modal_deposit(d, [&](int cc, int s, int i, int k, double v) {
-            unsafeAtomicAdd(&J[cc][mi(g, i, s, k)], (double)count(v) * kJqInv);
+    bool todo = dep;
+    for (int pass = 0;; pass++) {
+        DepWin W;
+        pin(d);
+        if (!deposit_window(todo, d, sred, sbox, W)) return;   // nothing (left) to deposit: uniform
+        const bool inside = todo && W.holds(d);
+        clear_window(W, sJ);
+        __syncthreads();
+        const int rl = threadIdx.x & (W.R - 1);
+        if (__all(!inside || same)) {   // the same for the whole wave: one path, not both
+            if (inside) {
+                const Corners n2 = W.corners(d.i2, d.k2, rl);
+                modal_deposit_same_cell(d, Count(), [&](int cc, int s, int di, int dk, long long v) {
+                    put(n2.w[di + 2 * dk] + 4 * (3 * cc + s), v);
+                });
+            }
+        } else if (inside) {
+            const Corners n1 = W.corners(d.i1, d.k1, rl), n2 = W.corners(d.i2, d.k2, rl);
+            modal_deposit(d, [&](int cc, int s, int h, int di, int dk, double a, double b) {
+                put((h ? n2 : n1).w[di + 2 * dk] + 4 * (3 * cc + s), Count()(a, b));
+            });
+        }
+        __syncthreads();
+        flush_window(g, W, sJ, J, [](long long v) { return (double)v * kJqInv; });
+        if (!W.box) return;
+        todo = todo && !inside;
+        if (__syncthreads_count(todo) <= kDepFew || pass == kDepPasses - 1) break;
+    }
+    if (todo)
+        modal_deposit(d, [&](int cc, int s, int h, int di, int dk, double a, double b) {
+            unsafeAtomicAdd(&J[cc][mi(g, (h ? d.i2 : d.i1) + di, s, (h ? d.k2 : d.k1) + dk)], (double)Count()(a, b) * kJqInv);
         });
-    const int cells = wi * wk;
-    int R = kDepCopies;
-    while (R > 1 && cells * R > kDepCells) R >>= 1;
-    const int rl = lane & (R - 1);
-    for (int e = threadIdx.x; e < 9 * cells * R; e += 256) sJ[e] = 0ull;
-    __syncthreads();
-    if (inside) {
-        auto add = [&](int cc, int s, int i, int k, long long cnt) {
-            atomicAdd(&sJ[((cc * 3 + s) * cells + (k - bkl) * wi + (i - bil)) * R + rl], (unsigned long long)cnt);
-        };
-        if (d.i1 == d.i2 && d.k1 == d.k2)
-            modal_deposit_same_cell(d, count, add);
-        else
-            modal_deposit(d, [&](int cc, int s, int i, int k, double v) { add(cc, s, i, k, count(v)); });
-    }
-    if (big) atomicOr(err, 2);
-    __syncthreads();
-    for (int e = threadIdx.x; e < 9 * cells; e += 256) {
-        long long v = 0;
-        for (int r = 0; r < R; r++) v += (long long)sJ[e * R + r];
-        if (v == 0) continue;
-        const int cs = e / cells, cell = e - cs * cells;
-        const int i = bil + cell % wi, k = bkl + cell / wi;
-        unsafeAtomicAdd(&J[cs / 3][mi(g, i, cs % 3, k)], (double)v * kJqInv);
-    }
 }
 
 __device__ inline uint64_t mix64d(uint64_t z)
