@@ -1236,22 +1236,15 @@ int pictor_step(pictor_ctx *c, int32_t nsteps)
     if (rc) return rc;
     if (c->pending_swap) return fail(PICTOR_ERR_ARG, "pictor_step inside a split step");
     if (c->cyl) {
+        if (c->cylm) return cylm_step(c, nsteps);
         // MAIN.F90:42-284 with the cylindrical routines
         for (int s = 0; s < nsteps; s++) {
             HIPTRY(hipEventRecord(c->ev[4], c->stream));
-            if (c->cylm) {
-                if ((rc = cylm_reset_current(c)) || (rc = cylm_b_half(c)) || (rc = cylm_push(c, true))) return rc;
-                if ((rc = cylm_exchange(c))) return rc;
-                if ((rc = cylm_b_half(c)) || (rc = cylm_e_phase(c, true, false)) || (rc = cylm_current_halo(c)) ||
-                    (rc = cylm_e_phase(c, false, true)) || (rc = cylm_window_after_step(c)))
-                    return rc;
-            } else {
-                if ((rc = cyl_reset_current(c)) || (rc = cyl_b_half(c)) || (rc = cyl_push(c, true))) return rc;
-                if ((rc = cyl_exchange(c))) return rc;
-                if ((rc = cyl_b_half(c)) || (rc = cyl_e_phase(c, true, false)) || (rc = cyl_current_halo(c)) ||
-                    (rc = cyl_e_phase(c, false, true)))
-                    return rc;
-            }
+            if ((rc = cyl_reset_current(c)) || (rc = cyl_b_half(c)) || (rc = cyl_push(c, true))) return rc;
+            if ((rc = cyl_exchange(c))) return rc;
+            if ((rc = cyl_b_half(c)) || (rc = cyl_e_phase(c, true, false)) || (rc = cyl_current_halo(c)) ||
+                (rc = cyl_e_phase(c, false, true)))
+                return rc;
             HIPTRY(hipEventRecord(c->ev[5], c->stream));
             HIPTRY(hipEventSynchronize(c->ev[5]));
             float ms = 0, f2 = 0;

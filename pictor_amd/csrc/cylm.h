@@ -53,7 +53,7 @@ struct CylmState {
     // (i, k) node, mx * mz nodes), rebuilt before every split push
     float4 *nf4 = nullptr;
     float2 *nf2 = nullptr;
-    int *d_err = nullptr;
+    int *d_err = nullptr;                // error bits; the first step of a run that raised one
     unsigned long long *d_count = nullptr;
     double *d_partial = nullptr;
     bool win_on = false;
@@ -83,4 +83,5 @@ int cylm_exchange(pictor_ctx *c);
 int cylm_inject(pictor_ctx *c, int nrp, int k0, int nzc, int ppc, unsigned long long seed, long long shift);
 int cylm_laser(pictor_ctx *c, double a0, double omega0, double tau, double w0, double zc);
 int cylm_window_after_step(pictor_ctx *c);
+int cylm_step(pictor_ctx *c, int nsteps);
 int cylm_diagnostics(pictor_ctx *c, double out[9]);

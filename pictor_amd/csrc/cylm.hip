@@ -540,6 +540,18 @@ __device__ inline void flush_window(const GridP &g, const DepWin &W, const T *sJ
     }
 }
 
+// the push's error flags; in a run of steps the first step that raises one closes the gates of
+// everything behind its push
+struct ModalErr {
+    int *bits = nullptr, *stop = nullptr;
+    Gate gate;
+    __device__ void raise(int b) const
+    {
+        atomicOr(bits, b);
+        if (stop) atomicMin(stop, gate.step);
+    }
+};
+
 // MoveDepositPrtl: gather, Boris, the local-frame move and rotation (cyl_movdep.F90:14-289),
 // then the modal deposit.  The particles keep the loader's cell order, so the 256 of a
 // block deposit into a small (i, k) window: it is accumulated in LDS and added to J once
@@ -552,8 +564,9 @@ __global__ __launch_bounds__(256) void k_cylm_push(GridP g, CylmP q, const doubl
                                                    const double *__restrict__ Bx, const double *__restrict__ By,
                                                    const double *__restrict__ Bz, double *__restrict__ Jx,
                                                    double *__restrict__ Jy, double *__restrict__ Jz, PartF64 P,
-                                                   long long n, int *__restrict__ err)
+                                                   long long n, ModalErr err)
 {
+    if (gate_closed(err.gate)) return;
     __shared__ __attribute__((aligned(16))) double sJ[kDepWords];
     __shared__ int sred[4][4], sbox[4];
     const long long m = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -594,7 +607,7 @@ __global__ __launch_bounds__(256) void k_cylm_push(GridP g, CylmP q, const doubl
         const double un = (X * u1 + Y * v1) * ir;
         const double vn = (-Y * u1 + X * v1) * ir;
         if (x1 >= g.mx - 3) {
-            atomicOr(err, 1);
+            err.raise(1);
         } else {
             dep = true;
             const double qthis = P.q[m] * q.qi;
@@ -671,8 +684,9 @@ __global__ __launch_bounds__(256) void k_cylm_nodes_f32(GridP g, const double *_
                                                         const double *__restrict__ Ey, const double *__restrict__ Ez,
                                                         const double *__restrict__ Bx, const double *__restrict__ By,
                                                         const double *__restrict__ Bz, float4 *__restrict__ nf4,
-                                                        float2 *__restrict__ nf2)
+                                                        float2 *__restrict__ nf2, Gate gate)
 {
+    if (gate_closed(gate)) return;
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (long long)g.mx * g.mz) return;
     const int i = 1 + (int)(t % g.mx), k = 1 + (int)(t / g.mx);
@@ -759,8 +773,9 @@ struct Count {
 __global__ __launch_bounds__(256) void k_cylm_push_split(GridP g, CylmP q, const float4 *__restrict__ nf4,
                                                          const float2 *__restrict__ nf2, double *__restrict__ Jx,
                                                          double *__restrict__ Jy, double *__restrict__ Jz, PartCylS P,
-                                                         long long n, int *__restrict__ err)
+                                                         long long n, ModalErr err)
 {
+    if (gate_closed(err.gate)) return;
     __shared__ __attribute__((aligned(16))) long long sJ[kDepWords];
     __shared__ int sred[4][4], sbox[4];
     const long long m = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -815,7 +830,7 @@ __global__ __launch_bounds__(256) void k_cylm_push_split(GridP g, CylmP q, const
         const float dth = atan2f(Y, X);
         const uint32_t t1 = t0 + (uint32_t)(unsigned long long)(long long)llrintf(dth * (float)(4294967296.0 / (2.0 * kPi)));
         if (i2 >= g.mx - 3) {
-            atomicOr(err, 1);
+            err.raise(1);
         } else {
             dep = true;
             const double qthis = (double)P.q[m] * q.qi * kJq;   // in counts: kJq is a power of two
@@ -855,7 +870,7 @@ __global__ __launch_bounds__(256) void k_cylm_push_split(GridP g, CylmP q, const
         if (!fits) {
             bool big = false;
             modal_deposit(d, [&](int, int, int, int, int, double a, double b) { big = big || !(fabs(a * b) <= L); });
-            if (big) atomicOr(err, 2);
+            if (big) err.raise(2);
         }
     }
     const bool same = d.i1 == d.i2 && d.k1 == d.k2;
@@ -929,8 +944,9 @@ __device__ inline void plasma_particle(const GridP &g, const CylmP &q, long long
 
 // appended at base + index
 __global__ void k_cylm_inject(GridP g, CylmP q, PartF64 P, long long base, int nrp, int k0, int nzc, int ppc,
-                              int epc, unsigned long long seed, long long shift)
+                              int epc, unsigned long long seed, long long shift, Gate gate)
 {
+    if (gate_closed(gate)) return;
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long total = (long long)nrp * nzc * ppc;
     if (t >= total) return;
@@ -944,8 +960,9 @@ __global__ void k_cylm_inject(GridP g, CylmP q, PartF64 P, long long base, int n
 }
 
 __global__ void k_cylm_inject_split(GridP g, CylmP q, PartCylS P, long long base, int nrp, int k0, int nzc, int ppc,
-                                    int epc, unsigned long long seed, long long shift)
+                                    int epc, unsigned long long seed, long long shift, Gate gate)
 {
+    if (gate_closed(gate)) return;
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long total = (long long)nrp * nzc * ppc;
     if (t >= total) return;
@@ -1003,8 +1020,9 @@ __global__ void k_cylm_shift_fields(GridP g, Ptrs6<double> P)
 }
 
 // particles: z -= 1; those below the window's start are dropped (flavour 0)
-__global__ void k_cylm_shift_particles(CylmP q, PartF64 P, long long n)
+__global__ void k_cylm_shift_particles(CylmP q, PartF64 P, long long n, Gate gate)
 {
+    if (gate_closed(gate)) return;
     const long long m = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= n || P.flv[m] == 0) return;
     const double z = P.z[m] - 1.0;
@@ -1013,8 +1031,9 @@ __global__ void k_cylm_shift_particles(CylmP q, PartF64 P, long long n)
 }
 
 // the same on the split record: k -= 1; a particle with k - 1 < zmin (z < zmin) is dropped
-__global__ void k_cylm_shift_split(CylmP q, PartCylS P, long long n)
+__global__ void k_cylm_shift_split(CylmP q, PartCylS P, long long n, Gate gate)
 {
+    if (gate_closed(gate)) return;
     const long long m = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= n) return;
     const uint32_t w = P.cell[m];
@@ -1168,6 +1187,212 @@ __global__ void k_cylm_compact_spans(R P, long long n, const long long *__restri
 #pragma unroll
     for (int j = 0; j < 4; j++)
         if (f[j]) P.copy_to(base + j, O, d++);
+}
+
+// ---- a step with open z ends (the moving window) in few launches ----
+// The separate kernels above read and write E four times and J three times a step, the axis, halo
+// and wall fills are launches of their own, and the window's shift copies E and B once more.
+// Here a thread owns one (i, s, k), i >= 4, all k, and finishes its point: the thread of i = 4 also
+// owns i = 1 .. 3, whose fills read nothing but its own values.  z ghosts (k <= 2, k >= mz - 2) and
+// the wall (i >= mx - 2) hold no field.  Memory-bound where the grid is large; a run of 61 steps at
+// 1024 x 128 took 315 us a step with the separate kernels (about 25 launches and two host waits a
+// step, the push 133 us of it) and takes 192, one of 41 at 4096 x 512 1861 and 1653.
+__device__ __forceinline__ bool zghost(const GridP &g, int k) { return k <= 2 || k >= g.mz - 2; }
+
+__device__ __forceinline__ void zero_j(const GridP &g, double *const *J, int i, int s, int k)
+{
+    for (int c = 0; c < 3; c++)
+        for (int ii = i == 4 ? 1 : i; ii <= i; ii++) J[c][mi(g, ii, s, k)] = 0.0;
+}
+
+// the fills of k_cylm_b_axis, k_cylm_zhalo and k_cylm_wall behind the update b of (i, s, k)
+__device__ __forceinline__ void finish_b(const GridP &g, const CylmP &q, double *const *B, const double *Ey, int i,
+                                         int s, int k, const double b[3])
+{
+    const long long o = mi(g, i, s, k);
+    const bool zero = zghost(g, k) || i >= g.mx - 2;
+    for (int c = 0; c < 3; c++) B[c][o] = zero ? 0.0 : b[c];
+    if (i != 4) return;
+    const double p = parity(s);
+    double b3[3] = {-(p * b[0]), 0.5 * (b[1] - p * b[1]), 0.0};
+    if (s == 0 && k <= g.mz - 1 && !zero) b3[2] = B[2][o - 1] - q.fld_halfc * (4.0 * q.inv_dr) * Ey[o];
+    else b3[2] = B[2][o - 1];
+    for (int c = 0; c < 3; c++) B[c][o - 1] = zero ? 0.0 : b3[c];
+    B[1][o - 2] = -(p * b[1]);
+    B[2][o - 2] = p * b[2];
+}
+
+// the arrays of the two kernels: F[0..2] = E, F[3..5] = B, F[6..8] = J, F[9..14] = shifted E and B
+struct CylF {
+    double *F[15];
+};
+
+// UpdateBfieldHalf and its fills; zero: ResetCurrent as well
+__global__ __launch_bounds__(256) void k_cylm_b_full(GridP g, CylmP q, CylF f, int zero, Gate gate)
+{
+    if (gate_closed(gate)) return;
+    const int ni = g.mx - 3;
+    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (long long)ni * 3 * g.mz) return;
+    const int i = 4 + (int)(t % ni);
+    t /= ni;
+    const int s = (int)(t % 3), k = 1 + (int)(t / 3);
+    const double *Ex = f.F[0], *Ey = f.F[1], *Ez = f.F[2];
+    const long long o = mi(g, i, s, k), sk = 3LL * g.mx, ss = g.mx;
+    double b[3] = {f.F[3][o], f.F[4][o], f.F[5][o]};
+    if (i <= g.mx - 3 && k <= g.mz - 1 && (i == 4 || !zghost(g, k))) {
+        const double h = q.fld_halfc, idr = q.inv_dr, idz = q.inv_dz;
+        const double r = rad(q, i), rph = r + 0.5 * q.dr, rp = r + q.dr;
+        const double dEz = s == 0 ? 0.0 : (s == 1 ? Ez[o + ss] : -Ez[o - ss]);
+        const double dEr = s == 0 ? 0.0 : (s == 1 ? Ex[o + ss] : -Ex[o - ss]);
+        b[0] = b[0] - h * dEz / r + h * idz * (Ey[o + sk] - Ey[o]);
+        b[1] = b[1] - h * idz * (Ex[o + sk] - Ex[o]) + h * idr * (Ez[o + 1] - Ez[o]);
+        b[2] = b[2] - h * (idr * (rp * Ey[o + 1] - r * Ey[o]) - dEr) / rph;
+    }
+    finish_b(g, q, f.F + 3, Ey, i, s, k, b);
+    if (zero) zero_j(g, f.F + 6, i, s, k);
+}
+
+// the Lehe form: k_cylm_update_b_lehe_col's columns over all k; rows 1, mz - 1 and mz take no update
+template <int KC>
+__global__ __launch_bounds__(256) void k_cylm_b_full_lehe(GridP g, CylmP q, CylF f, int zero, Gate gate)
+{
+    if (gate_closed(gate)) return;
+    const int ni = g.mx - 3, nk = g.mz - 3, nkc = (nk + KC - 1) / KC;
+    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (long long)ni * 3 * nkc) return;
+    const int i = 4 + (int)(t % ni);
+    t /= ni;
+    const int s = (int)(t % 3), ch = (int)(t / 3);
+    const int kb = 2 + KC * ch, ke = min(kb + KC, 2 + nk);
+    const double *Ex = f.F[0], *Ey = f.F[1], *Ez = f.F[2];
+    double *const *B = f.F + 3;
+    auto plain = [&](int k) {
+        const long long o = mi(g, i, s, k);
+        const double b[3] = {B[0][o], B[1][o], B[2][o]};
+        finish_b(g, q, B, Ey, i, s, k, b);
+        if (zero) zero_j(g, f.F + 6, i, s, k);
+    };
+    if (ch == 0) plain(1);
+    if (ch == nkc - 1) { plain(g.mz - 1); plain(g.mz); }
+    if (i >= g.mx - 2) {
+        for (int k = kb; k < ke; k++) plain(k);
+        return;
+    }
+    const double h = q.fld_halfc, idr = q.inv_dr, idz = q.inv_dz;
+    const double r = rad(q, i), rph = r + 0.5 * q.dr, rp = r + q.dr;
+    double xa[4], ya[4], yb[3], za[3], zb[3], xt[3], zt[3];
+    auto row3 = [&](int m, int j) {
+        const long long o = mi(g, i, s, m);
+        yb[j] = Ey[o + 1]; za[j] = Ez[o]; zb[j] = Ez[o + 1];
+        xt[j] = dth(g, Ex, o, s); zt[j] = dth(g, Ez, o, s);
+    };
+    auto row4 = [&](int m, int j) {
+        const long long o = mi(g, i, s, m);
+        xa[j] = Ex[o]; ya[j] = Ey[o];
+    };
+    for (int j = 0; j < 3; j++) row3(kb - 1 + j, j);
+    for (int j = 0; j < 4; j++) row4(kb - 1 + j, j);
+    for (int k = kb; k < ke; k++) {
+        const long long o = mi(g, i, s, k);
+        const double gtz = q.l_tt * zt[1] + q.l_tz * zt[2] + q.l_tz * zt[0];
+        const double gzy = q.l_zz * (ya[2] - ya[1]) + q.l_zd * (ya[3] - ya[0]);
+        const double gzx = q.l_zz * (xa[2] - xa[1]) + q.l_zd * (xa[3] - xa[0]);
+        const double grz = q.l_rr * (zb[1] - za[1]) + q.l_rz * (zb[2] - za[2]) + q.l_rz * (zb[0] - za[0]);
+        const double gr1y = q.l_rr * (rp * yb[1] - r * ya[1]) + q.l_rz * (rp * yb[2] - r * ya[2])
+                            + q.l_rz * (rp * yb[0] - r * ya[0]);
+        const double gtx = q.l_tt * xt[1] + q.l_tz * xt[2] + q.l_tz * xt[0];
+        const double b[3] = {B[0][o] - h * gtz / r + h * idz * gzy, B[1][o] - h * idz * gzx + h * idr * grz,
+                             B[2][o] - h * (idr * gr1y - gtx) / rph};
+        finish_b(g, q, B, Ey, i, s, k, b);
+        if (zero) zero_j(g, f.F + 6, i, s, k);
+        if (k + 1 < ke) {
+            for (int j = 0; j < 2; j++) {
+                yb[j] = yb[j + 1]; za[j] = za[j + 1]; zb[j] = zb[j + 1]; xt[j] = xt[j + 1]; zt[j] = zt[j + 1];
+            }
+            for (int j = 0; j < 3; j++) { xa[j] = xa[j + 1]; ya[j] = ya[j + 1]; }
+            row3(k + 2, 2);
+            row4(k + 3, 3);
+        }
+    }
+}
+
+// UpdateEfield, AxisCurrentBC, AddCurrent and their fills.  SHIFT: the window advances by a cell
+// behind this step; E and B go one row back into the second buffers (fills included), J is cleared.
+template <bool SHIFT>
+__global__ __launch_bounds__(256) void k_cylm_e_full(GridP g, CylmP q, CylF f, Gate gate)
+{
+    if (gate_closed(gate)) return;
+    const int ni = g.mx - 3;
+    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (long long)ni * 3 * g.mz) return;
+    const int i = 4 + (int)(t % ni);
+    t /= ni;
+    const int s = (int)(t % 3), k = 1 + (int)(t / 3);
+    double *const *E = f.F, *const *B = f.F + 3, *const *J = f.F + 6;
+    const long long o = mi(g, i, s, k), sk = 3LL * g.mx, ss = g.mx;
+    const bool zero = zghost(g, k) || i >= g.mx - 2;
+    double e[3] = {0.0, 0.0, 0.0}, j[3] = {0.0, 0.0, 0.0}, bo[3] = {0.0, 0.0, 0.0};
+    if (i == 4) {   // AxisCurrentBC, on every row
+        for (int c = 0; c < 3; c++) j[c] = J[c][o];
+        j[1] = j[1] - J[1][o - 1];
+        j[2] = j[2] - J[2][o - 1];
+        if (!SHIFT) {
+            J[1][o] = j[1];
+            J[2][o] = j[2];
+            J[0][o - 1] = 0.0;
+            J[1][o - 2] = 0.0;
+            J[2][o - 2] = 0.0;
+        }
+    }
+    if (!zero) {
+        if (i != 4)
+            for (int c = 0; c < 3; c++) j[c] = J[c][o];
+        const double fldc = q.fldc, idr = q.inv_dr, idz = q.inv_dz;
+        const double r = rad(q, i), rp = r + 0.5 * q.dr, rm = r - 0.5 * q.dr;
+        const double *Bx = B[0], *By = B[1], *Bz = B[2];
+        const double dBz = s == 0 ? 0.0 : (s == 1 ? Bz[o + ss] : -Bz[o - ss]);
+        const double dBr = s == 0 ? 0.0 : (s == 1 ? Bx[o + ss] : -Bx[o - ss]);
+        bo[0] = Bx[o]; bo[1] = By[o]; bo[2] = Bz[o];
+        e[0] = E[0][o] + fldc * dBz / rp - fldc * idz * (bo[1] - By[o - sk]);
+        e[1] = E[1][o] + fldc * idz * (bo[0] - Bx[o - sk]) - fldc * idr * (bo[2] - Bz[o - 1]);
+        e[2] = E[2][o] + fldc * idr * (rp * bo[1] - rm * By[o - 1]) / r - fldc * dBr / r;
+        const double th = s == 0 ? 2.0 * kPi : kPi;
+        e[0] = e[0] - j[0] * q.inv_dz / (rp * th);
+        e[1] = e[1] - j[1] * q.inv_dr * q.inv_dz / th;
+        e[2] = e[2] - j[2] * q.inv_dr / (r * th);
+    }
+    const double p = parity(s);
+    const double e3[3] = {0.5 * (e[0] - p * e[0]), -(p * e[1]), p * e[2]};
+    if (!SHIFT) {
+        for (int c = 0; c < 3; c++) E[c][o] = e[c];
+        if (i == 4) {
+            for (int c = 0; c < 3; c++) E[c][o - 1] = zero ? 0.0 : e3[c];
+            E[0][o - 2] = -(p * e[0]);
+        }
+        return;
+    }
+    // row k goes to k - 1; rows mz - 3 .. mz (from k = mz - 2 .. mz and 1) hold nothing
+    const int kd = k == 1 ? g.mz : k - 1;
+    const bool empty = k == 1 || k >= g.mz - 2, ghost = empty || zghost(g, kd);
+    const long long od = mi(g, i, s, kd);
+    double *const *E2 = f.F + 9, *const *B2 = f.F + 12;
+    for (int c = 0; c < 3; c++) {
+        E2[c][od] = ghost ? 0.0 : e[c];
+        B2[c][od] = ghost ? 0.0 : bo[c];
+    }
+    if (i == 4) {
+        for (int c = 0; c < 3; c++) {
+            E2[c][od - 1] = ghost ? 0.0 : e3[c];
+            B2[c][od - 1] = ghost ? 0.0 : B[c][o - 1];
+            for (int a = 2; a <= 3; a++) {   // i = 2, 1
+                E2[c][od - a] = empty ? 0.0 : E[c][o - a];
+                B2[c][od - a] = empty ? 0.0 : B[c][o - a];
+            }
+        }
+        E2[0][od - 2] = -(p * (empty ? 0.0 : e[0]));
+    }
+    zero_j(g, J, i, s, k);
 }
 
 void fields(pictor_ctx *c, double *E[3], double *B[3], double *J[3])
@@ -1413,7 +1638,7 @@ int cylm_setup(pictor_ctx *c)
 {
     CylmState &st = c->cm;
     if (!st.d_err) {
-        HIPTRY(dalloc(&st.d_err, 1));
+        HIPTRY(dalloc(&st.d_err, 2));
         HIPTRY(dalloc(&st.d_count, 1));
         HIPTRY(dalloc(&st.d_partial, 3 * 1024));
         HIPTRY(hipMemsetAsync(st.d_err, 0, sizeof(int), c->stream));
@@ -1569,11 +1794,10 @@ int cylm_reset_current(pictor_ctx *c)
     return PICTOR_OK;
 }
 
-int cylm_push(pictor_ctx *c, bool timed)
+static int cylm_enqueue_push(pictor_ctx *c, const ModalErr &err)
 {
     double *E[3], *B[3], *J[3];
     fields(c, E, B, J);
-    if (timed) HIPTRY(hipEventRecord(c->ev[0], c->stream));
     if (c->np > 0 && split_form(c)) {
         CylmState &st = c->cm;
         const long long nodes = (long long)c->g.mx * c->g.mz;
@@ -1582,15 +1806,32 @@ int cylm_push(pictor_ctx *c, bool timed)
             HIPTRY(dalloc(&st.nf2, nodes));
         }
         hipLaunchKernelGGL(k_cylm_nodes_f32, blocks_of(nodes), dim3(256), 0, c->stream, c->g, E[0], E[1], E[2], B[0],
-                           B[1], B[2], st.nf4, st.nf2);
+                           B[1], B[2], st.nf4, st.nf2, err.gate);
         hipLaunchKernelGGL(k_cylm_push_split, blocks_of(c->np), dim3(256), 0, c->stream, c->g, c->cq, st.nf4, st.nf2,
-                           J[0], J[1], J[2], st.ps, c->np, st.d_err);
+                           J[0], J[1], J[2], st.ps, c->np, err);
     } else if (c->np > 0)
         hipLaunchKernelGGL(k_cylm_push, blocks_of(c->np), dim3(256), 0, c->stream, c->g, c->cq, E[0], E[1], E[2], B[0],
-                           B[1], B[2], J[0], J[1], J[2], c->pcyl, c->np, c->cm.d_err);
+                           B[1], B[2], J[0], J[1], J[2], c->pcyl, c->np, err);
+    return PICTOR_OK;
+}
+
+int cylm_push(pictor_ctx *c, bool timed)
+{
+    if (timed) HIPTRY(hipEventRecord(c->ev[0], c->stream));
+    int rc = cylm_enqueue_push(c, ModalErr{c->cm.d_err, nullptr, Gate{}});
+    if (rc) return rc;
     if (timed) HIPTRY(hipEventRecord(c->ev[1], c->stream));
     HIPTRY(hipGetLastError());
     c->pending_swap = true;
+    return PICTOR_OK;
+}
+
+static int cylm_error(int err)
+{
+    if (err & 1) return fail(PICTOR_ERR_BOUNDS, "modal cylinder: a particle reached the outer wall");
+    if (err & 2)
+        return fail(PICTOR_ERR_CAPACITY, "modal cylinder, split form: a current contribution above 64 charge cells "
+                                         "(the fixed-point range); use the FP64 form");
     return PICTOR_OK;
 }
 
@@ -1602,11 +1843,20 @@ int cylm_exchange(pictor_ctx *c)
     c->pending_swap = false;
     // the flags report this push only: clear them for the next one
     if (err) HIPTRY(hipMemsetAsync(c->cm.d_err, 0, sizeof(int), c->stream));
-    if (err & 1) return fail(PICTOR_ERR_BOUNDS, "modal cylinder: a particle reached the outer wall");
-    if (err & 2)
-        return fail(PICTOR_ERR_CAPACITY, "modal cylinder, split form: a current contribution above 64 charge cells "
-                                         "(the fixed-point range); use the FP64 form");
-    return PICTOR_OK;
+    return cylm_error(err);
+}
+
+// the particles of nrp x nzc cells behind the np slots in use: room for them is the caller's
+static void launch_inject(pictor_ctx *c, int nrp, int k0, int nzc, int ppc, unsigned long long seed, long long shift,
+                          Gate gate)
+{
+    const long long add = (long long)nrp * nzc * ppc;
+    if (split_form(c))
+        hipLaunchKernelGGL(k_cylm_inject_split, blocks_of(add), dim3(256), 0, c->stream, c->g, c->cq, c->cm.ps, c->np,
+                           nrp, k0, nzc, ppc, c->cfg.epc, seed, shift, gate);
+    else
+        hipLaunchKernelGGL(k_cylm_inject, blocks_of(add), dim3(256), 0, c->stream, c->g, c->cq, c->pcyl, c->np, nrp,
+                           k0, nzc, ppc, c->cfg.epc, seed, shift, gate);
 }
 
 int cylm_inject(pictor_ctx *c, int nrp, int k0, int nzc, int ppc, unsigned long long seed, long long shift)
@@ -1618,12 +1868,7 @@ int cylm_inject(pictor_ctx *c, int nrp, int k0, int nzc, int ppc, unsigned long 
     if (rc) return rc;
     const long long add = (long long)nrp * nzc * ppc;
     if ((rc = ensure_room(c, add))) return rc;
-    if (split_form(c))
-        hipLaunchKernelGGL(k_cylm_inject_split, blocks_of(add), dim3(256), 0, c->stream, g, c->cq, c->cm.ps, c->np, nrp,
-                           k0, nzc, ppc, c->cfg.epc, seed, shift);
-    else
-        hipLaunchKernelGGL(k_cylm_inject, blocks_of(add), dim3(256), 0, c->stream, g, c->cq, c->pcyl, c->np, nrp, k0,
-                           nzc, ppc, c->cfg.epc, seed, shift);
+    launch_inject(c, nrp, k0, nzc, ppc, seed, shift, Gate{});
     HIPTRY(hipGetLastError());
     c->np += add;
     return PICTOR_OK;
@@ -1658,6 +1903,15 @@ int cylm_window_after_step(pictor_ctx *c)
     return rc;
 }
 
+static void launch_shift_particles(pictor_ctx *c, Gate gate)
+{
+    if (c->np > 0 && split_form(c))
+        hipLaunchKernelGGL(k_cylm_shift_split, blocks_of(c->np), dim3(256), 0, c->stream, c->cq, c->cm.ps, c->np, gate);
+    else if (c->np > 0)
+        hipLaunchKernelGGL(k_cylm_shift_particles, blocks_of(c->np), dim3(256), 0, c->stream, c->cq, c->pcyl, c->np,
+                           gate);
+}
+
 static int cylm_window_shifts(pictor_ctx *c)
 {
     CylmState &st = c->cm;
@@ -1676,10 +1930,7 @@ static int cylm_window_shifts(pictor_ctx *c)
         double *E[3], *B[3], *J[3];
         fields(c, E, B, J);
         launch_fill_zero_n<double>(J, 3, c->g.ncell, c->stream);
-        if (c->np > 0 && split_form(c))
-            hipLaunchKernelGGL(k_cylm_shift_split, blocks_of(c->np), dim3(256), 0, c->stream, c->cq, c->cm.ps, c->np);
-        else if (c->np > 0)
-            hipLaunchKernelGGL(k_cylm_shift_particles, blocks_of(c->np), dim3(256), 0, c->stream, c->cq, c->pcyl, c->np);
+        launch_shift_particles(c, Gate{});
         st.win_shift += 1;
         int rc = PICTOR_OK;
         if (st.win_nrp > 0 && st.win_ppc > 0 &&
@@ -1688,6 +1939,159 @@ static int cylm_window_shifts(pictor_ctx *c)
         if ((rc = cylm_field_halo(c, 0)) || (rc = cylm_field_halo(c, 1))) return rc;
     }
     return PICTOR_OK;
+}
+
+// MAIN.F90:42-284 with the modal routines, one host wait a step
+static int cylm_step_plain(pictor_ctx *c)
+{
+    int rc;
+    HIPTRY(hipEventRecord(c->ev[4], c->stream));
+    if ((rc = cylm_reset_current(c)) || (rc = cylm_b_half(c)) || (rc = cylm_push(c, true))) return rc;
+    if ((rc = cylm_exchange(c))) return rc;
+    if ((rc = cylm_b_half(c)) || (rc = cylm_e_phase(c, true, false)) || (rc = cylm_current_halo(c)) ||
+        (rc = cylm_e_phase(c, false, true)) || (rc = cylm_window_after_step(c)))
+        return rc;
+    HIPTRY(hipEventRecord(c->ev[5], c->stream));
+    HIPTRY(hipEventSynchronize(c->ev[5]));
+    float ms = 0, f2 = 0;
+    if (hipEventElapsedTime(&ms, c->ev[0], c->ev[1]) == hipSuccess) { c->t_ms[0] += ms; c->t_n[0]++; }
+    if (hipEventElapsedTime(&f2, c->ev[4], c->ev[5]) == hipSuccess) { c->t_ms[2] += f2; c->t_n[2]++; }
+    return PICTOR_OK;
+}
+
+// what a step that did not run has to give back
+struct CylMark {
+    long long np, win_steps, win_shift, since_sort;
+    int swaps;
+};
+
+// Open z ends: up to kRun steps enqueued together (until a sort or an injection that needs room is
+// due), then one wait.  A push that raises an error closes the gates of all that follows it; the
+// host takes back what it had noted for those steps, so that the state is the one behind that push,
+// as it is when the host looks at the flags of every step.
+static int cylm_run_open(pictor_ctx *c, int nsteps, int &done)
+{
+    constexpr int kRun = 32;
+    CylmState &st = c->cm;
+    hipStream_t s = c->stream;
+    const GridP &g = c->g;
+    while (c->sev.size() < 3 * kRun + 1) {
+        hipEvent_t e;
+        HIPTRY(hipEventCreate(&e));
+        c->sev.push_back(e);
+    }
+    int m = std::min(kRun, nsteps - done);
+    if (st.sort_period > 0) m = (int)std::min<long long>(m, std::max<long long>(1, st.sort_period - st.steps_since_sort));
+    CylF f;
+    auto load = [&]() {
+        for (int i = 0; i < 3; i++) {
+            f.F[i] = (double *)c->E[i]; f.F[3 + i] = (double *)c->B[i]; f.F[6 + i] = (double *)c->J[i];
+            f.F[9 + i] = (double *)c->E2[i]; f.F[12 + i] = (double *)c->B2[i];
+        }
+    };
+    auto swap = [&]() {
+        for (int i = 0; i < 3; i++) { std::swap(c->E[i], c->E2[i]); std::swap(c->B[i], c->B2[i]); }
+    };
+    const long long pts = (long long)(g.mx - 3) * 3 * g.mz;
+    constexpr int KC = 8;
+    const long long cols = (long long)(g.mx - 3) * 3 * ((g.mz - 3 + KC - 1) / KC);
+    auto b_half = [&](int zero, Gate gate) {
+        load();
+        if (c->cq.lehe)
+            hipLaunchKernelGGL((k_cylm_b_full_lehe<KC>), blocks_of(cols), dim3(256), 0, s, g, c->cq, f, zero, gate);
+        else
+            hipLaunchKernelGGL(k_cylm_b_full, blocks_of(pts), dim3(256), 0, s, g, c->cq, f, zero, gate);
+    };
+    std::vector<CylMark> mark;
+    bool inject_late = false, clear = false;
+    int swaps = 0;
+    HIPTRY(hipMemsetAsync(st.d_err + 1, 0x7f, sizeof(int), s));
+    int t = 0;
+    for (; t < m && !inject_late; t++) {
+        const Gate before{st.d_err + 1, t}, behind{st.d_err + 1, t + 1};
+        HIPTRY(hipEventRecord(c->sev[3 * t], s));
+        b_half(clear ? 0 : 1, before);   // a shift has cleared J
+        HIPTRY(hipEventRecord(c->sev[3 * t + 1], s));
+        int rc = cylm_enqueue_push(c, ModalErr{st.d_err, st.d_err + 1, before});
+        if (rc) return rc;
+        HIPTRY(hipEventRecord(c->sev[3 * t + 2], s));
+        mark.push_back({c->np, st.win_steps, st.win_shift, st.steps_since_sort, swaps});
+        b_half(0, behind);
+        st.win_steps += 1;
+        clear = (double)st.win_steps * c->ph.c >= (double)(st.win_shift + 1);
+        if (clear) {
+            hipLaunchKernelGGL(k_cylm_e_full<true>, blocks_of(pts), dim3(256), 0, s, g, c->cq, f, behind);
+            swap();
+            swaps++;
+            launch_shift_particles(c, behind);
+            st.win_shift += 1;
+            if (st.win_nrp > 0 && st.win_ppc > 0) {
+                const long long add = (long long)st.win_nrp * st.win_ppc;
+                inject_late = c->np + add > st.cap;
+                if (!inject_late) {
+                    launch_inject(c, st.win_nrp, g.mz - 3, 1, st.win_ppc, st.win_seed, st.win_shift, behind);
+                    c->np += add;
+                }
+            }
+        } else {
+            hipLaunchKernelGGL(k_cylm_e_full<false>, blocks_of(pts), dim3(256), 0, s, g, c->cq, f, behind);
+        }
+        st.steps_since_sort += st.sort_period > 0 ? 1 : 0;
+    }
+    HIPTRY(hipGetLastError());
+    HIPTRY(hipEventRecord(c->sev[3 * t], s));
+    HIPTRY(hipMemcpyAsync(c->h_flags, st.d_err, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
+    HIPTRY(hipStreamSynchronize(s));
+    const int err = c->h_flags[0], ran = err ? c->h_flags[1] : t;
+    float ms = 0;
+    for (int k = 0; k < ran; k++) {
+        if (hipEventElapsedTime(&ms, c->sev[3 * k + 1], c->sev[3 * k + 2]) == hipSuccess) { c->t_ms[0] += ms; c->t_n[0]++; }
+        if (hipEventElapsedTime(&ms, c->sev[3 * k], c->sev[3 * k + 3]) == hipSuccess) { c->t_ms[2] += ms; c->t_n[2]++; }
+    }
+    if (err) {
+        const CylMark &k = mark[ran];
+        c->np = k.np;
+        st.win_steps = k.win_steps;
+        st.win_shift = k.win_shift;
+        st.steps_since_sort = k.since_sort;
+        if ((swaps - k.swaps) & 1) swap();
+        HIPTRY(hipMemsetAsync(st.d_err, 0, sizeof(int), s));
+        return cylm_error(err);
+    }
+    done += t;
+    const bool sort = st.sort_period > 0 && st.steps_since_sort >= st.sort_period;
+    if (!inject_late && !sort) return PICTOR_OK;
+    int rc = PICTOR_OK;
+    HIPTRY(hipEventRecord(c->ev[4], s));
+    if (inject_late) rc = cylm_inject(c, st.win_nrp, g.mz - 3, 1, st.win_ppc, st.win_seed, st.win_shift);
+    if (!rc && sort) rc = cylm_sort(c);
+    if (rc) return rc;
+    HIPTRY(hipEventRecord(c->ev[5], s));
+    HIPTRY(hipEventSynchronize(c->ev[5]));
+    if (hipEventElapsedTime(&ms, c->ev[4], c->ev[5]) == hipSuccess) c->t_ms[2] += ms;   // the last step's
+    return rc;
+}
+
+int cylm_step(pictor_ctx *c, int nsteps)
+{
+    CylmState &st = c->cm;
+    int rc = cylm_setup(c);
+    // the open-ended run: a second set of E and B to shift into, and at most one shift a step
+    bool open = c->cq.zopen && st.win_on && c->ph.c < 1.0;
+    for (int i = 0; i < 3 && open; i++)
+        open = (c->E2[i] || dalloc((double **)&c->E2[i], c->g.ncell) == hipSuccess) &&
+               (c->B2[i] || dalloc((double **)&c->B2[i], c->g.ncell) == hipSuccess);
+    if (c->cq.zopen && !open) (void)hipGetLastError();
+    for (int done = 0; done < nsteps && !rc;) {
+        const bool one = (double)(st.win_steps + 1) * c->ph.c < (double)(st.win_shift + 2);
+        if (open && one) {
+            rc = cylm_run_open(c, nsteps, done);
+        } else {
+            rc = cylm_step_plain(c);
+            done++;
+        }
+    }
+    return rc;
 }
 
 int cylm_diagnostics(pictor_ctx *c, double out[9])

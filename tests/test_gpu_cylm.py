@@ -628,3 +628,93 @@ def test_current_does_not_depend_on_the_particle_order(form, n):
                 # the crowded nodes take up to 0.3 n contributions in another order: 2^-53 of each partial sum
                 assert np.abs(a - b).max() <= max(n, 10) * 2.0 ** -53 * 20.0 * np.abs(a).max()
     assert np.abs(J[0][0]).max() > 0.0
+
+
+@pytest.mark.parametrize("form", ["fp32_split", "fp64"])
+@pytest.mark.parametrize("fdtd", ["yee", "lehe"])
+@pytest.mark.parametrize("nr,nz", [(8, 8), (24, 13), (70, 41)])
+def test_open_run_equals_phases_and_shifts(form, fdtd, nr, nz):
+    # steps of a window run enqueued together against the phase calls, with the window's shift made by
+    # hand: every row moves one cell back, the front and the z ghosts restart at zero, J is cleared,
+    # E's axis rows follow from the fourth column.  The first fields fill ghosts and wall, too.
+    say(f"[case] cylm open run {form} {fdtd} {nr}x{nz}")
+    c, steps = 0.4, 7
+    rng = np.random.default_rng(nr + nz)
+
+    def make():
+        sim = Simulation(nr, 2, nz, ndim=3, epc=4, c=c, c_ompe=10.0, form=form, geometry="cyl_modal", fdtd=fdtd)
+        sim.moving_window(True)
+        return sim
+
+    with make() as sim:
+        shape = sim.shape
+    n = 40 * nz
+    P = dict(q=rng.uniform(0.5, 1.0, n), x=rng.uniform(4.0, nr - 0.5, n),
+             y=rng.uniform(0.0, 2.0 * np.pi, n), z=rng.uniform(3.0, nz + 2.9, n), u=rng.normal(0.0, 0.02, n),
+             v=rng.normal(0.0, 0.2, n), w=rng.normal(0.0, 0.3, n), flv=np.full(n, 2, np.int32))
+    F0 = [np.asfortranarray(1e-3 * rng.standard_normal(shape)) for _ in FIELDS]
+    with make() as a, make() as b:
+        for sim in (a, b):
+            sim.upload_fields(*F0)
+            sim.upload_particles(**P)
+        a.step(steps)
+        got = a.download_fields()
+        pa = a.download_particles()
+        shift = 0
+        for t in range(1, steps + 1):
+            b.step_phases()
+            if t * c < shift + 1:
+                continue
+            shift += 1
+            f, p = b.download_fields(), b.download_particles()
+            mx, mz = shape[0], shape[2]
+            for k in FIELDS:
+                g = np.zeros(shape, order="F")
+                g[:, :, :mz - 4] = f[k][:, :, 1:mz - 3]
+                f[k] = g
+            par = np.array([1.0, -1.0, -1.0])[:, None]
+            four = {k: f[k][3].copy() for k in ("Ex", "Ey", "Ez")}
+            f["Ex"][2], f["Ex"][1] = 0.5 * (four["Ex"] - par * four["Ex"]), -par * four["Ex"]
+            f["Ey"][2], f["Ez"][2] = -par * four["Ey"], par * four["Ez"]
+            for k in FIELDS:
+                f[k][2:mx - 3, :, :2] = 0.0
+                f[k][2:mx - 3, :, mz - 3:] = 0.0
+                f[k][mx - 3:] = 0.0
+            p["z"] = np.where(p["flv"] != 0, p["z"] - 1.0, p["z"])
+            p["flv"] = np.where(p["z"] < 3.0, 0, p["flv"]).astype(np.int32)
+            b.upload_fields(*[f[k] for k in FIELDS])
+            b.upload_particles(**p)
+            b.ResetCurrent()
+        want, pb = b.download_fields(), b.download_particles()
+    live = pa["flv"] != 0
+    assert live.sum() == (pb["flv"] != 0).sum()
+    for k in ("Ex", "Ey", "Ez", "Bx", "By", "Bz", "Jx", "Jy", "Jz"):
+        if form == "fp32_split":
+            assert np.array_equal(got[k], want[k]), k
+        else:   # the order of the current's FP64 adds
+            assert np.abs(got[k] - want[k]).max() <= 1e-12 * max(np.abs(want[k]).max(), 1e-300), k
+    for k in ("x", "z", "u", "w"):
+        assert np.abs(pa[k][live] - pb[k][pb["flv"] != 0]).max() <= (0.0 if form == "fp32_split" else 1e-12), k
+
+
+@pytest.mark.parametrize("form", ["fp32_split", "fp64"])
+def test_error_inside_an_open_run_stops_behind_that_push(form):
+    # a particle that reaches the wall in step 4: the same error and state as steps one at a time
+    say(f"[case] cylm open run error {form}")
+    P = dict(q=[1.0, 1.0], x=[19.5, 9.5], y=[0.0, 1.0], z=[20.5, 20.5], u=[3.0, 0.0], v=[0.0, 0.0], w=[0.0, 0.1],
+             flv=np.array([2, 2], np.int32))
+    out = []
+    for one in (False, True):
+        with Simulation(18, 2, 32, ndim=3, epc=4, c=0.4, c_ompe=10.0, form=form, geometry="cyl_modal") as sim:
+            sim.moving_window(True)
+            sim.upload_particles(**P)
+            with pytest.raises(RuntimeError, match="outer wall"):
+                for _ in range(12 if one else 1):
+                    sim.step(1 if one else 12)
+            out.append((sim.download_fields(), sim.download_particles(), sim.timer("step")[1]))
+    (fa, pa, na), (fb, pb, nb) = out
+    assert na == nb and 0 < na < 12
+    for k in fa:
+        assert np.array_equal(fa[k], fb[k]), k
+    for k in pa:
+        assert np.array_equal(pa[k], pb[k]), k
