@@ -30,8 +30,11 @@ void launch_eng_push(const AdjP &ap, const void *nE, const void *nB, EPart<R> in
 template <typename R>
 void launch_eng_adjoint(const AdjP &ap, const void *nE, const void *nB, EPart<R> st, double *const Eb[3],
                         EPart<R> adj, double *const gE[3], double *const gB[3], long long n, hipStream_t s);
-void launch_node_to_stag(const AdjP &ap, double *const gE[3], double *const gB[3], double *const Eb[3],
-                         double *const Bb[3], hipStream_t s);
+// the field parts of a reverse step, before and behind the particles' part (Bn: the new Bb)
+void launch_adj_before(const AdjP &ap, const PhysP &ph, double *const Eb[3], double *const Bb[3], double *const gE[3],
+                       double *const gB[3], long long ncell, hipStream_t s);
+void launch_adj_behind(const AdjP &ap, const PhysP &ph, double *const Eb[3], double *const Bb[3], double *const gE[3],
+                       double *const gB[3], double *const Bn[3], hipStream_t s);
 template <typename R>
 void launch_eng_load(const AdjP &ap, const double *const raw[6], const int *flv, EPart<R> out, long long n, int *err,
                      hipStream_t s);

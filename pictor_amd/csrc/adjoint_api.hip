@@ -13,10 +13,11 @@
 //    The push records for every input slot the slot its particle went to, and
 //    the reverse step walks the same bins (adjoint_fast.hip).  The field work of
 //    a step is one launch (kernels_fieldstep.hip), which writes the E and B that
-//    the next push reads straight into the arrays the reverse sweep keeps.  Recomputed states hold the same particles
-//    as the forward pass's, possibly in another order inside a bin (slot
-//    reservation order varies between runs); the particle ids map the
-//    adjoint from one to the other at segment boundaries.
+//    the next push reads straight into the arrays the reverse sweep keeps.
+//    Recomputed states hold the same particles as the forward pass's, possibly
+//    in another order inside a bin (slot reservation order varies between
+//    runs); the particle ids map the adjoint from one to the other at segment
+//    boundaries.
 //  * unsorted (both forms): particles in the caller's order, one thread per
 //    particle, node fields of every step (adjoint.hip).
 #include <hip/hip_runtime.h>
@@ -209,7 +210,7 @@ struct AdjEngine : AdjEngineBase {
     // FP32 split form: the low part of E (E = hi + lo), as the context keeps it
     float *Elo[3] = {};
     std::vector<float *> ckElo;
-    double *Eb[3] = {}, *Bb[3] = {}, *gE[3] = {}, *gB[3] = {};
+    double *Eb[3] = {}, *Bb[3] = {}, *Bn[3] = {}, *gE[3] = {}, *gB[3] = {};
     // current filter (curr_filter > 0): scratch, and the filtered adjoint current
     // the particle reverse step reads (Jadj = Ebf, else Eb)
     double *Jt[3] = {}, *Ebf[3] = {};
@@ -270,7 +271,7 @@ struct AdjEngine : AdjEngineBase {
     {
         if (c && c->stream) (void)hipStreamSynchronize(c->stream);
         for (int i = 0; i < 3; i++) {
-            E[i] = B[i] = nullptr; J[i] = Eb[i] = Bb[i] = gE[i] = gB[i] = nullptr;
+            E[i] = B[i] = nullptr; J[i] = Eb[i] = Bb[i] = Bn[i] = gE[i] = gB[i] = nullptr;
             Jt[i] = Ebf[i] = Jadj[i] = nullptr;
             Elo[i] = nullptr;
             E2[i] = B2[i] = nullptr; Elo2[i] = nullptr; J2[i] = nullptr;
@@ -317,7 +318,7 @@ struct AdjEngine : AdjEngineBase {
         ap.jscale = ctx_jscale;
         for (int i = 0; i < 3; i++) {
             HIPTRY(mem.get(&E[i], ncell)); HIPTRY(mem.get(&B[i], ncell)); HIPTRY(mem.get(&J[i], ncell));
-            HIPTRY(mem.get(&Eb[i], ncell)); HIPTRY(mem.get(&Bb[i], ncell));
+            HIPTRY(mem.get(&Eb[i], ncell)); HIPTRY(mem.get(&Bb[i], ncell)); HIPTRY(mem.get(&Bn[i], ncell));
             HIPTRY(mem.get(&gE[i], ncell)); HIPTRY(mem.get(&gB[i], ncell));
             if (c->curr_filter > 0) { HIPTRY(mem.get(&Jt[i], ncell)); HIPTRY(mem.get(&Ebf[i], ncell)); }
             Jadj[i] = c->curr_filter > 0 ? Ebf[i] : Eb[i];
@@ -649,13 +650,7 @@ struct AdjEngine : AdjEngineBase {
     {
         hipStream_t s = c->stream;
         const GridP &g = c->g;
-        PhysP pa = c->ph, pb = c->ph;
-        pa.fld_halfc = -c->ph.fldc;      // B-half kernel as the transpose of the E update's curl
-        pb.fldc = -c->ph.fld_halfc;      // E kernel (curl only) as the transpose of a B half step
-        launch_ghost_copy<double>(g, Eb, s);
-        launch_update_b_half<double>(g, pa, Eb, Bb, s);
-        double *gEB[6] = {gE[0], gE[1], gE[2], gB[0], gB[1], gB[2]};
-        launch_fill_zero_n<double>(gEB, 6, ncell, s);
+        launch_adj_before(ap, c->ph, Eb, Bb, gE, gB, ncell, s);
         if (c->curr_filter > 0) {
             // the adjoint current is F^T(-jscale Eb) = F(-jscale Eb): the periodic 1-2-1
             // filter is symmetric; its ghosts are the images (the fold's transpose)
@@ -664,13 +659,8 @@ struct AdjEngine : AdjEngineBase {
             launch_ghost_copy<double>(g, Ebf, s);
         }
         particle_adjoint();
-        launch_ghost_copy<double>(g, Bb, s);
-        launch_update_e<double>(g, pb, Eb, Bb, s);
-        launch_current_fold<double>(g, gE, s, gB);
-        launch_ghost_copy<double>(g, gE, s, gB);
-        launch_node_to_stag(ap, gE, gB, Eb, Bb, s);
-        launch_ghost_copy<double>(g, Bb, s);
-        launch_update_e<double>(g, pb, Eb, Bb, s);
+        launch_adj_behind(ap, c->ph, Eb, Bb, gE, gB, Bn, s);
+        std::swap_ranges(Bb, Bb + 3, Bn);
         HIPTRY(hipGetLastError());
         return PICTOR_OK;
     }
