@@ -559,7 +559,7 @@ int step_periodic(pictor_ctx *c, int nsteps)
             HIPTRY(hipEventRecord(c->sev[2 * t + 2], s));
             c->cur = 1 - c->cur;
             double *J[3] = {(double *)c->J[0], (double *)c->J[1], (double *)c->J[2]};
-            if (last || filter) launch_current_fold<double>(c->g, J, s, nullptr, gate);
+            if (last || filter) launch_current_fold<double>(c->g, J, s, gate);
             if (filter) launch_smoothen_current(c->g, c->curr_filter, J, c->Jt, s, gate);
             FieldStepP<R> P = field_args<R>(c, in_place);
             P.fold = !(last || filter);

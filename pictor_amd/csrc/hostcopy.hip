@@ -103,6 +103,26 @@ bool grow(HostRing &r, int want)
     return true;
 }
 
+// an array in memory that the device reaches (the caller's pinned or managed memory): straight into it
+hipError_t deliver_mapped(const HostItem &it, hipStream_t s, bool &done)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, it.dst) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipSuccess;
+    }
+    if (a.type == hipMemoryTypeUnregistered || !a.devicePointer) return hipSuccess;
+    done = true;
+    if (it.kind == HostItem::kRaw) return hipMemcpyAsync(it.dst, it.src, it.n * it.elem, hipMemcpyDefault, s);
+    constexpr size_t per = 1 << 26;   // elements of a launch
+    for (size_t o = 0; o < it.n; o += per) {
+        const Piece p{&it, o, std::min(per, it.n - o), 0};
+        const hipError_t e = enqueue(p, (char *)a.devicePointer + o * it.elem, s);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 // without pinned memory: the runtime's own copies, converted pieces through a device chunk
 hipError_t deliver_plain(const std::vector<Piece> &todo, hipStream_t s)
 {
@@ -141,6 +161,10 @@ hipError_t deliver(HostRing &ring, const std::vector<HostItem> &items, hipStream
     std::vector<Batch> batch;
     size_t bytes = 0, used = kChunk;   // of the last batch
     for (const HostItem &it : items) {
+        bool direct = false;
+        const hipError_t d = deliver_mapped(it, s, direct);
+        if (d != hipSuccess) return d;
+        if (direct) continue;
         const size_t per = kChunk / it.elem;
         for (size_t o = 0; o < it.n; o += per) {
             Piece p{&it, o, std::min(per, it.n - o), 0};

@@ -503,9 +503,9 @@ void launch_ghost_copy(const GridP &g, R *const F[3], hipStream_t s, R *const G[
 }
 
 template <typename JT>
-void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, JT *const K[3], Gate gate)
+void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, Gate gate)
 {
-    Ptrs6<JT> P{{J[0], J[1], J[2], K ? K[0] : nullptr, K ? K[1] : nullptr, K ? K[2] : nullptr}};
+    Ptrs6<JT> P{{J[0], J[1], J[2]}};
     int naxes = (g.ndim == 3) ? 3 : 2;
     for (int a = 0; a < naxes; a++) {
         if (!g.per[a]) continue;   // null neighbours: the ghost current stays where it is
@@ -513,7 +513,7 @@ void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, JT *cons
         if (a != 0) ext[0] = g.mx - 5;
         ext[a] = 5;
         long long total = ext[0] * ext[1] * ext[2];
-        hipLaunchKernelGGL(k_current_fold<JT>, dim3(nblocks(total, 256), K ? 2 : 1), dim3(256), 0, s, g, a, P, gate);
+        hipLaunchKernelGGL(k_current_fold<JT>, dim3(nblocks(total, 256)), dim3(256), 0, s, g, a, P, gate);
     }
 }
 
@@ -630,7 +630,7 @@ template void launch_add_current<float, double>(const GridP &, const PhysP &, fl
                                                 double, hipStream_t);
 template void launch_ghost_copy<double>(const GridP &, double *const[3], hipStream_t, double *const[3]);
 template void launch_ghost_copy<float>(const GridP &, float *const[3], hipStream_t, float *const[3]);
-template void launch_current_fold<double>(const GridP &, double *const[3], hipStream_t, double *const[3], Gate);
+template void launch_current_fold<double>(const GridP &, double *const[3], hipStream_t, Gate);
 template void launch_fill_zero_n<double>(double *const *, int, long long, hipStream_t);
 template void launch_fill_zero_n<float>(float *const *, int, long long, hipStream_t);
 template void launch_copy_n<float>(float *const *, float *const *, int, long long, hipStream_t, Gate);

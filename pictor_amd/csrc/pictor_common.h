@@ -180,11 +180,11 @@ template <typename T>
 struct Ptrs6 {
     T *p[6];
 };
-// G / K: an optional second set of three arrays treated in the same launch
+// G: an optional second set of three arrays treated in the same launch
 template <typename R>
 void launch_ghost_copy(const GridP &g, R *const F[3], hipStream_t s, R *const G[3] = nullptr);
 template <typename JT>
-void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, JT *const K[3] = nullptr, Gate gate = Gate{});
+void launch_current_fold(const GridP &g, JT *const J[3], hipStream_t s, Gate gate = Gate{});
 template <typename T>
 void launch_fill_zero(T *p, long long n, hipStream_t s);
 template <typename T>

@@ -6,6 +6,7 @@ import threading
 
 import numpy as np
 import pytest
+import torch
 
 from pictor_amd import Simulation, setup_weibel
 from pictor_amd._lib import check, lib
@@ -70,6 +71,24 @@ def test_particles(form, n, epc):
     for k in ("x", "y"):
         assert np.abs(out[k][o] - P[k]).max() <= (0.0 if form == "fp64" else 2.0 ** -24), k
     assert out["tile"].min() >= 0 and out["tile"].max() > 0
+
+
+@pytest.mark.parametrize("form", ["fp32_split", "fp64"])
+def test_pinned_destination(form):
+    # the caller's pinned arrays take the results without the ring, beside pageable ones
+    say(form)
+    with Simulation(168, 160, form=form) as sim:
+        sim.upload_fields(*_fields(sim, 4))
+        want = sim.download_fields()
+        n = int(np.prod(sim.shape))
+        pin = [torch.full((n,), float("nan"), dtype=torch.float64, pin_memory=True) for _ in range(4)]
+        page = np.full(sim.shape, np.nan, order="F")
+        dp = ctypes.POINTER(ctypes.c_double)
+        ptr = [ctypes.cast(t.data_ptr(), dp) for t in pin] + [page.ctypes.data_as(dp)] + [None] * 4
+        check(lib().pictor_download_fields(sim._ctx, *ptr))
+        for name, t in zip(F, pin):
+            assert np.array_equal(t.numpy().reshape(sim.shape, order="F"), want[name]), name
+        assert np.array_equal(page, want["By"])
 
 
 def test_threads():
