@@ -24,12 +24,13 @@
 //
 // What bounds the loop (2048 x 2048, 268M particles, tile 16): in the split form the vector
 // ALU is busy 82 % of the cycles and LDS 74 %, at 1.8 GHz, so instructions and LDS accesses
-// are what counts: the field is staged as bilinear coefficients (18 multiply-adds a gather),
-// a thread keeps its bin between iterations, a node count is one fused multiply-add
-// (count_of), the destination follows from the tile-local cell, and one LDS add reserves the
-// slots of a wave.  A thread loads its next particle before it pushes the current one and
-// waits for it before the stores (settle): a wait behind them would last until they are
-// done.  Push 3.40 -> 3.09 ms (11.4 ps per particle); at 1024 x 1024 in FP64, where the
+// are what counts: a thread keeps its bin between iterations, a node count is a product and one
+// add (count_of), the destination follows from the tile-local cell, and one LDS add reserves the
+// slots of a wave.  (Bilinear coefficients in LDS, six products fewer a gather, and counts by one
+// fused multiply-add took 3.06 ms too, and rounded otherwise than the reverse step.)  A thread
+// loads its next particle before it pushes the current one and waits for it before the stores
+// (settle): a wait behind them would last until they are
+// done.  Push 3.40 -> 3.06 ms (11.4 ps per particle); at 1024 x 1024 in FP64, where the
 // record's 120 B move at 4.4 TB/s, 1.87 -> 1.81 ms, and at 256 x 256 in FP64 (tile 8, four
 // workgroups per CU, latency) 104 -> 87 us.
 #include "pictor_common.h"
@@ -335,9 +336,8 @@ __global__ __launch_bounds__(BS) void k_push2d_split(GridP g, PhysP ph, TileP tp
     constexpr int WW = W * W;
     constexpr int MB = 18;   // species (<= 2) x 9 directions
     constexpr int kLogT = T == 8 ? 3 : (T == 16 ? 4 : 5);
-    // field of the tile's cells: cell lc holds 6 float4, component c of the reference's
-    // VecE/VecB(nn, cell) (movdep_routines.F90:6-223) as the coefficients (a, b, c, d) of its
-    // bilinear form a + b x + y (c + d x)
+    // field of the tile's cells: cell lc holds 6 float4, component c at corners 1..4 (the
+    // reference's VecE/VecB(nn, cell), movdep_routines.F90:6-223)
     __shared__ float4 sC[6 * T * T];
     __shared__ unsigned long long sJ[3][WW];
     __shared__ int sStart[MB + 1], sVs[MB];
@@ -387,10 +387,7 @@ __global__ __launch_bounds__(BS) void k_push2d_split(GridP g, PhysP ph, TileP tp
             v[5][cn] = (Bz[p - 1 - mx] + Bz[p - 1] + Bz[p - mx] + Bz[p]) * 0.25f + bz0;
         }
 #pragma unroll
-        for (int cc = 0; cc < 6; cc++) {
-            const float bx = v[cc][1] - v[cc][0], by = v[cc][3] - v[cc][2];
-            sC[6 * lc + cc] = make_float4(v[cc][0], bx, v[cc][2] - v[cc][0], by - bx);
-        }
+        for (int cc = 0; cc < 6; cc++) sC[6 * lc + cc] = make_float4(v[cc][0], v[cc][1], v[cc][2], v[cc][3]);
     }
     for (int e = tid; e < WW; e += BS) { sJ[0][e] = 0ull; sJ[1][e] = 0ull; sJ[2][e] = 0ull; }
     __syncthreads();
@@ -449,7 +446,11 @@ __global__ __launch_bounds__(BS) void k_push2d_split(GridP g, PhysP ph, TileP tp
                 const int lc = (jj0 - 2) * T + (ii0 - 2);
                 const float4 gEx = sC[6 * lc], gEy = sC[6 * lc + 1], gEz = sC[6 * lc + 2];
                 const float4 gBx = sC[6 * lc + 3], gBy = sC[6 * lc + 4], gBz = sC[6 * lc + 5];
-                auto at = [&](const float4 &g) { return (g.x + g.y * x0 + y0 * (g.z + g.w * x0)) * qm; };
+                // the weighted sum of push_fwd (adjoint_math.h), term for term: the reverse step
+                // recomputes this one and has to round as it did
+                const float w1 = (1.0f - x0) * (1.0f - y0), w2 = x0 * (1.0f - y0);
+                const float w3 = (1.0f - x0) * y0, w4 = x0 * y0;
+                auto at = [&](const float4 &g) { return (w1 * g.x + w2 * g.y + w3 * g.z + w4 * g.w) * qm; };
                 const float pEx = at(gEx), pEy = at(gEy), pEz = at(gEz);
                 const float hBx = at(gBx), hBy = at(gBy), hBz = at(gBz);
                 // Boris, movdep.F90:143-173 (hardware rsq/rcp: about 1 ulp, FP32 form)

@@ -104,13 +104,13 @@ __device__ inline int norm_dir(int dd, int n)
 // |v| < 2^31, so one conversion)
 __device__ inline int quanti(float v) { return (int)__builtin_rintf(v); }
 
-// F * W as a count: rounded to the nearest integer (ties to even) by adding 1.5 * 2^52,
-// whose sum's bit pattern minus the constant's is that integer for |F W| < 2^51.
+// F * W, a product in FP64, as a count: rounded to the nearest integer (ties to even) by adding
+// 1.5 * 2^52, whose sum's bit pattern minus the constant's is that integer for |F W| < 2^51.
 constexpr double kCountBias = 6755399441055744.0;
 constexpr unsigned long long kCountBits = 0x4338000000000000ull;
 __device__ inline unsigned long long count_of(double F, double W)
 {
-    return (unsigned long long)__double_as_longlong(__builtin_fma(F, W, kCountBias)) - kCountBits;
+    return (unsigned long long)__double_as_longlong(F * W + kCountBias) - kCountBits;
 }
 
 // The two zigzag half-segments of the 2-D split form (movdep.F90:177-237)
