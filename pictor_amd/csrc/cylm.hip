@@ -745,18 +745,17 @@ __device__ inline void gather_nodes(const GridP &g, const float4 *__restrict__ n
         }
 }
 
-// the count rint(a b) (a in counts) as a 64-bit integer: |a b| <= 64 kJq = 2^42, and adding
-// 1.5 2^52 rounds it to an integer in the low mantissa bits (ties to even, as rint)
+// the count rint(a b) (a in counts, a b a product in FP64) as a 64-bit integer: |a b| <= 64 kJq =
+// 2^42, and adding 1.5 2^52 rounds it to an integer in the low mantissa bits (ties to even, as rint)
 struct Count {
-    __device__ static double bias() { return 6755399441055744.0; }
-    __device__ long long operator()(double a, double b) const
+    __device__ static unsigned long long bits(double a, double b)
     {
-        return __double_as_longlong(__builtin_fma(a, b, bias())) - 0x4338000000000000LL;
+        return (unsigned long long)__double_as_longlong(a * b + 6755399441055744.0);
     }
+    __device__ long long operator()(double a, double b) const { return (long long)(bits(a, b) - 0x4338000000000000ULL); }
     __device__ long long operator()(double a1, double b1, double a2, double b2) const
     {
-        return __double_as_longlong(__builtin_fma(a1, b1, bias())) +
-               (__double_as_longlong(__builtin_fma(a2, b2, bias())) - (long long)0x8670000000000000ULL);
+        return (long long)(bits(a1, b1) + (bits(a2, b2) - 0x8670000000000000ULL));
     }
 };
 
@@ -767,9 +766,10 @@ struct Count {
 // Flags: 1 = a particle reached the wall, 2 = a contribution above 64 charge cells (the
 // fixed-point range).
 // Bound by the VALU (75 % of its issue slots, 830 instructions a wave).  31.5 million particles,
-// 4096 x 512 cells, with the node copy: 1451 -> 1077 us.  The range check on the factors, not on
-// each of 44 contributions, one FMA per count, immediate LDS offsets and further windows for a block
-// over the end of a row gave it; 8 accumulator copies; 4 take 2 % longer.
+// 4096 x 512 cells, with the node copy: 1451 -> 1088 us.  The range check on the factors, not on
+// each of 44 contributions, immediate LDS offsets and further windows for a block
+// over the end of a row gave it; 8 accumulator copies; 4 take 2 % longer.  (Counts by one fused
+// multiply-add, one rounding for two: 1 % faster and other bits.)
 __global__ __launch_bounds__(256) void k_cylm_push_split(GridP g, CylmP q, const float4 *__restrict__ nf4,
                                                          const float2 *__restrict__ nf2, double *__restrict__ Jx,
                                                          double *__restrict__ Jy, double *__restrict__ Jz, PartCylS P,
