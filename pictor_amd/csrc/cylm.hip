@@ -372,7 +372,7 @@ __device__ inline void modal_deposit(const DepMove &d, Add add)
 
 // modal_deposit for a particle that stays in its cell (i1 = i2, k1 = k2): both r-z
 // half-segments land on the same nodes; add(component, slot, di, dk, value) gets their sum,
-// term(a1, b1, a2, b2)
+// term(a1, b1, a2, b2).  For the counts of the split form, which add exactly in any order.
 template <class Term, class Add>
 __device__ inline void modal_deposit_same_cell(const DepMove &d, Term term, Add add)
 {
@@ -406,12 +406,6 @@ __device__ inline void pin(DepMove &d)
     pin(d.wx); pin(d.wz); pin(d.pt[0]); pin(d.pt[1]); pin(d.pt[2]);
 }
 
-// a contribution in FP64
-struct Product {
-    __device__ double operator()(double a, double b) const { return a * b; }
-    __device__ double operator()(double a1, double b1, double a2, double b2) const { return a1 * b1 + a2 * b2; }
-};
-
 // minimum over the wave, in every lane: row shifts and broadcasts (DPP), no LDS traffic
 __device__ inline int wave_min(int v)
 {
@@ -429,14 +423,14 @@ __device__ inline int wave_max(int v) { return ~wave_min(~v); }
 
 // mode cells of the block's deposit window held in LDS: 9 accumulators (3 components x
 // 3 slots) per (i, k) cell, FP64 or 64-bit counts.  A window of at most kDepCells / R cells keeps
-// R = 2, 4 or kDepCopies copies of its accumulators (lane l adds into copy l % R): the particles of
+// R = 2, 4 or 8 copies of its accumulators (lane l adds into copy l % R): the particles of
 // one cell sit in adjacent lanes and would otherwise serialise on the same LDS words.
 // Copy r of a cell is slot L = cell R + r; its accumulator cs = 3 component + slot is word
 // 36 (L / 4) + 4 cs + L % 4: the nine of a node are immediate offsets of one address (an address
 // each cost the split push a quarter of its time in 32-bit multiplies), and the copies of 8 (R = 4)
 // neighbouring cells cover the 64 banks once.
 constexpr int kDepCells = 448;
-constexpr int kDepCopies = 8;
+constexpr int kDepCopies = 8, kDepCopiesF64 = 4;
 constexpr int kDepWords = 9 * kDepCells;
 // words of the nodes (di, dk) of a cell: w[di + 2 dk]
 struct Corners {
@@ -462,15 +456,17 @@ struct DepWin {
 // when the block's particles spread wider than kDepCells cells (a block whose sorted particles run
 // over the end of a row of cells and into the next; electrons expelled, crossing the axis or trapped
 // in the wake, far from their array neighbours), the window is a box of kBoxI x kBoxK cells around the
-// block's first depositing particle, and those outside it go through another window, up to kDepPasses.
-// The last kDepFew or fewer add to J directly: a row of cells is 30 blocks at 480 x 16 particles, and
-// with everything outside the first box added directly the block over its end made the push 20 %
-// slower.
+// block's first depositing particle.  Split form: those outside it go through another window, up to
+// kDepPasses, and the last kDepFew or fewer add to J directly: a row of cells is 30 blocks at 480 x 16
+// particles, and with everything outside the first box added directly the block over its end made the
+// push 20 % slower.  FP64: those outside add to J directly.  There the sums are rounded, so how they
+// are grouped shows in the fields: the order of the adds of a node in a block, four copies and the box
+// keep that grouping the same in every version of this push.
 constexpr int kDepPasses = 4, kDepFew = 16;
 constexpr int kBoxI = 28, kBoxK = 4;
 
-// the block's deposit window; uniform over the block; false: no particle deposits
-__device__ inline bool deposit_window(bool dep, const DepMove &d, int (*sred)[4], int *sbox, DepWin &W)
+// the block's deposit window with at most `copies` copies; uniform over the block; false: no particle deposits
+__device__ inline bool deposit_window(bool dep, const DepMove &d, int copies, int (*sred)[4], int *sbox, DepWin &W)
 {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int ilo = wave_min(dep ? min(d.i1, d.i2) : INT_MAX), ihi = wave_max(dep ? max(d.i1, d.i2) : INT_MIN);
@@ -506,7 +502,7 @@ __device__ inline bool deposit_window(bool dep, const DepMove &d, int (*sred)[4]
     W.wi = __builtin_amdgcn_readfirstlane(W.wi);
     W.wk = __builtin_amdgcn_readfirstlane(W.wk);
     const int cells = W.wi * W.wk;
-    W.R = kDepCopies;                           // cells R <= kDepCells
+    W.R = copies;                               // cells R <= kDepCells
     while (W.R > 1 && cells * W.R > kDepCells) W.R >>= 1;
     return true;
 }
@@ -532,7 +528,7 @@ __device__ inline void flush_window(const GridP &g, const DepWin &W, const T *sJ
         const T *a = sJ + DepWin::word((k * W.wi + i) * W.R) + 4 * cs;
         T v = a[0];
         if (W.R > 1) v += a[1];
-        if (W.R > 2) v += a[2] + a[3];
+        if (W.R > 2) { v += a[2]; v += a[3]; }
         if (W.R > 4) v += a[36] + a[37] + a[38] + a[39];
         if (v == 0) continue;
         const int cc = (cs * 11) >> 5;          // cs / 3
@@ -556,9 +552,9 @@ struct ModalErr {
 // then the modal deposit.  The particles keep the loader's cell order, so the 256 of a
 // block deposit into a small (i, k) window: it is accumulated in LDS and added to J once
 // per cell and accumulator.  Bound by FP64 and address arithmetic (VALU) with 4 waves per SIMD:
-// 1.57 million particles, 1024 x 128 cells, 170 -> 133 us with one address per node, the DPP
-// reductions, a single path per wave and, for a particle that stays in its cell, 28 LDS adds
-// instead of 36.
+// 1.57 million particles, 1024 x 128 cells, 149 -> 141 us with one address per node and the DPP
+// reductions.  (One LDS add for both halves of a move inside a cell, eight copies and a window for
+// the particles outside the first take 122 us, and regroup rounded sums.)
 __global__ __launch_bounds__(256) void k_cylm_push(GridP g, CylmP q, const double *__restrict__ Ex,
                                                    const double *__restrict__ Ey, const double *__restrict__ Ez,
                                                    const double *__restrict__ Bx, const double *__restrict__ By,
@@ -637,41 +633,25 @@ __global__ __launch_bounds__(256) void k_cylm_push(GridP g, CylmP q, const doubl
         P.x[m] = x1; P.y[m] = tn; P.z[m] = zn;
         P.u[m] = un; P.v[m] = vn; P.w[m] = wn;
     }
-    const bool same = d.i1 == d.i2 && d.k1 == d.k2;
     double *J[3] = {Jx, Jy, Jz};
-    bool todo = dep;
-    for (int pass = 0;; pass++) {
-        DepWin W;
-        pin(d);
-        if (!deposit_window(todo, d, sred, sbox, W)) return;   // nothing (left) to deposit: uniform
-        const bool inside = todo && W.holds(d);
-        clear_window(W, sJ);
-        __syncthreads();
-        const int rl = threadIdx.x & (W.R - 1);
-        if (__all(!inside || same)) {   // the same for the whole wave: one path, not both
-            if (inside) {
-                const Corners n2 = W.corners(d.i2, d.k2, rl);
-                modal_deposit_same_cell(d, Product(),
-                                        [&](int cc, int s, int di, int dk, double v) {
-                                            atomicAdd(sJ + n2.w[di + 2 * dk] + 4 * (3 * cc + s), v);
-                                        });
-            }
-        } else if (inside) {
-            const Corners n1 = W.corners(d.i1, d.k1, rl), n2 = W.corners(d.i2, d.k2, rl);
-            modal_deposit(d, [&](int cc, int s, int h, int di, int dk, double a, double b) {
-                atomicAdd(sJ + (h ? n2 : n1).w[di + 2 * dk] + 4 * (3 * cc + s), a * b);
-            });
-        }
-        __syncthreads();
-        flush_window(g, W, sJ, J, [](double v) { return v; });
-        if (!W.box) return;
-        todo = todo && !inside;
-        if (__syncthreads_count(todo) <= kDepFew || pass == kDepPasses - 1) break;
-    }
-    if (todo)
+    DepWin W;
+    if (!deposit_window(dep, d, kDepCopiesF64, sred, sbox, W)) return;   // nothing to deposit: uniform
+    const bool inside = dep && W.holds(d);
+    if (dep && !inside)
         modal_deposit(d, [&](int cc, int s, int h, int di, int dk, double a, double b) {
             unsafeAtomicAdd(&J[cc][mi(g, (h ? d.i2 : d.i1) + di, s, (h ? d.k2 : d.k1) + dk)], a * b);
         });
+    clear_window(W, sJ);
+    __syncthreads();
+    if (inside) {
+        const int rl = threadIdx.x & (W.R - 1);
+        const Corners n1 = W.corners(d.i1, d.k1, rl), n2 = W.corners(d.i2, d.k2, rl);
+        modal_deposit(d, [&](int cc, int s, int h, int di, int dk, double a, double b) {
+            atomicAdd(sJ + (h ? n2 : n1).w[di + 2 * dk] + 4 * (3 * cc + s), a * b);
+        });
+    }
+    __syncthreads();
+    flush_window(g, W, sJ, J, [](double v) { return v; });
 }
 
 // The node-centred FP32 copy of E and B that the split push gathers from, rebuilt before
@@ -880,7 +860,7 @@ __global__ __launch_bounds__(256) void k_cylm_push_split(GridP g, CylmP q, const
     for (int pass = 0;; pass++) {
         DepWin W;
         pin(d);
-        if (!deposit_window(todo, d, sred, sbox, W)) return;   // nothing (left) to deposit: uniform
+        if (!deposit_window(todo, d, kDepCopies, sred, sbox, W)) return;   // nothing (left) to deposit: uniform
         const bool inside = todo && W.holds(d);
         clear_window(W, sJ);
         __syncthreads();

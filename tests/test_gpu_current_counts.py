@@ -98,3 +98,39 @@ def test_modal_counts(shuffled):
     for name, want in (("Jx", Jr), ("Jz", Jz)):
         got = F[name][:, 0, :] * 2.0 ** 36      # slot 0: mode m = 0
         assert np.array_equal(got, want), (name, np.count_nonzero(got != want))
+
+
+@pytest.mark.parametrize("n", [1, 7, 64])
+def test_modal_fp64_sums_in_order(n):
+    # FP64 sums show their order.  One wave of particles has one: lane l adds into copy l % 4, one node
+    # after the other, first and second half of the move apart, and the copies are added 0 to 3
+    say("modal FP64 sums,", n, "particles")
+    nr = nz = 32
+    rng = np.random.default_rng(n)
+    P = {"q": -rng.uniform(1.0, 400.0, n), "x": 12.0 + rng.uniform(0.0, 2.0, n), "y": rng.uniform(0.0, 2 * np.pi, n),
+         "z": 14.0 + rng.uniform(0.0, 2.0, n), "u": rng.normal(0, 0.7, n), "v": rng.normal(0, 0.7, n),
+         "w": rng.normal(0, 0.7, n)}
+    with Simulation(nr, 2, nz, ndim=3, epc=16, c=0.8, c_ompe=20.0, mi_me=1e30, form="fp64", geometry="cyl_modal",
+                    dr=4.0) as sim:
+        sim.upload_particles(**P, flv=np.full(n, 2, np.int32))
+        sim.ResetCurrent()
+        sim.MoveDepositPrtl()
+        sim.ExchangePrtl()
+        now = sim.download_particles()
+        F = sim.download_fields()
+        qi = sim.qi
+    x0, z0, x1, z1 = P["x"], P["z"], now["x"], now["z"]
+    i0, k0, i1, k1 = (np.floor(p).astype(int) for p in (x0, z0, x1, z1))
+    qs = P["q"] * qi
+    xr, zr = _relay(x0, x1, i0.astype(float), i1.astype(float)), _relay(z0, z1, k0.astype(float), k1.astype(float))
+    J = np.zeros((2, 4, nr + 5, nz + 5))
+    for xa, za, xb, zb, i, k in ((x0, z0, xr, zr, i0, k0), (xr, zr, x1, z1, i1, k1)):
+        Fx, Fz = qs * (xb - xa), qs * (zb - za)
+        Wx, Wz = 0.5 * (xa + xb) - i, 0.5 * (za + zb) - k
+        for c, di, dk, v in ((0, 0, 0, Fx * (1.0 - Wz)), (0, 0, 1, Fx * Wz), (1, 0, 0, Fz * (1.0 - Wx)), (1, 1, 0, Fz * Wx)):
+            for l in range(n):
+                J[c, l % 4, i[l] + di - 1, k[l] + dk - 1] += v[l]
+    for c, name in enumerate(("Jx", "Jz")):
+        want = ((J[c, 0] + J[c, 1]) + J[c, 2]) + J[c, 3]
+        assert np.count_nonzero(want) > 0
+        assert np.array_equal(F[name][:, 0, :], want), np.abs(F[name][:, 0, :] - want).max()
