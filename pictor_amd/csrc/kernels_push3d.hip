@@ -113,6 +113,7 @@ __global__ __launch_bounds__(BS) void k_push3d_f64(GridP g, PhysP ph, TileP tp, 
             const int ip0 = (int)x0, jp0 = (int)y0, kp0 = (int)z0;
             // node-window coordinates of the cell (origin i0-1)
             const int gi = ip0 - (i0 - 1), gj = jp0 - (j0 - 1), gk = kp0 - (k0 - 1);
+            xn = x0; yn = y0; zn = z0;   // a particle refused below stays where it is
             if (gi < 0 || gi > T + 1 || gj < 0 || gj > T + 1 || gk < 0 || gk > T + 1 || flv < 1 || flv > ph.nflvr) {
                 flag_error(sp, kErrBounds);
                 d = 13;
