@@ -40,9 +40,12 @@ constexpr int kUseUnsorted = -101;   // internal: the FP64 tile bins do not fit,
 // Device memory of an engine.  A forward and backward pass needs a few hundred arrays (16.7 GB
 // in all at 512 x 512 over 200 steps); allocating and freeing each of them took 63 ms of a 70 ms
 // pass at 128 x 128 in FP64 and 85 ms of 225 at 512 x 512.  The engine cuts them from chunks
-// that it keeps for its next pass: reset() starts over, trim() gives back the chunks that the
-// pass did not reach, and the destructor of the engine (pictor_adjoint_release, the context's
-// end) gives back all.  A pass of the same sizes cuts the same arrays from the same chunks.
+// that it keeps for its next pass, each array from the first chunk with room for it: reset() starts
+// over, trim() gives back the chunks that the pass cut nothing from, and the destructor of the
+// engine (pictor_adjoint_release, the context's end) gives back all.  A pass of the same sizes cuts
+// the same arrays from the same chunks.  Where the card is full, chunks not cut from go first; a
+// pass that still finds no room is repeated with separate(): every array an allocation of its own,
+// as if nothing had been kept.
 class Arena {
 public:
     ~Arena() { release(); }
@@ -52,52 +55,97 @@ public:
         *p = nullptr;
         // large arrays on 2 MiB boundaries, as separate allocations are: packed closer, the push
         // over 57 MB arrays takes 12 % longer (512 x 512: forward 32.0 against 35.8 ms)
-        const size_t raw = std::max<size_t>(n, 1) * sizeof(T), align = raw >= (16u << 20) ? 2u << 20 : 256;
+        const size_t raw = std::max<size_t>(n, 1) * sizeof(T), align = raw >= kLarge ? 2u << 20 : 256;
         const size_t bytes = (raw + align - 1) / align * align;
-        if (align > 256) used_ = (used_ + align - 1) / align * align;
-        while (at_ < chunks_.size() && used_ + bytes > chunks_[at_].size) { at_++; used_ = 0; }
-        if (at_ == chunks_.size()) {
-            // doubling chunks: few allocations, at most half of the last one unused
-            const size_t want = std::max(bytes, std::min<size_t>(std::max<size_t>(total_, 1 << 20), 1 << 30));
-            Chunk c{nullptr, want};
-            hipError_t e = hipMalloc((void **)&c.p, c.size);
-            if (e != hipSuccess && want > bytes) {
-                (void)hipGetLastError();
-                c.size = bytes;
-                e = hipMalloc((void **)&c.p, c.size);
-            }
-            if (e != hipSuccess) return e;
-            chunks_.push_back(c);
-            total_ += c.size;
-            used_ = 0;
+        for (Chunk &c : chunks_)
+            if (cut(c, bytes, align, (void **)p)) return hipSuccess;
+        // doubling chunks for small arrays, a whole number of arrays of this size for large ones
+        // (most come in sixes): few allocations, little left over
+        size_t want = bytes;
+        if (!separate_ && bytes < kChunk)
+            want = raw >= kLarge ? kChunk / bytes * bytes
+                                 : std::max(bytes, std::min<size_t>(std::max<size_t>(total_, 1 << 20), kChunk));
+        Chunk c{nullptr, want, 0};
+        hipError_t e = take(c);
+        if (e != hipSuccess && want > bytes) {
+            c.size = bytes;
+            e = take(c);
         }
-        *p = (T *)(chunks_[at_].p + used_);
-        used_ += bytes;
+        if (e != hipSuccess && drop_unused()) e = take(c);
+        failed_ = failed_ || e != hipSuccess;
+        if (e != hipSuccess) return e;
+        total_ += c.size;
+        chunks_.push_back(c);
+        cut(chunks_.back(), bytes, align, (void **)p);
         return hipSuccess;
     }
-    void reset() { at_ = 0; used_ = 0; }
-    void trim()
+    // memory beside the arena for the length of a call (dfree gives it back)
+    template <typename T>
+    hipError_t get_beside(T **p, size_t n)
     {
-        const size_t keep = chunks_.empty() ? 0 : at_ + 1;
-        while (chunks_.size() > keep) {
-            total_ -= chunks_.back().size;
-            (void)hipFree(chunks_.back().p);
-            chunks_.pop_back();
+        hipError_t e = dalloc(p, n);
+        if (e == hipSuccess) return e;
+        (void)hipGetLastError();
+        if (drop_unused() && (e = dalloc(p, n)) != hipSuccess) (void)hipGetLastError();
+        if (e != hipSuccess) {
+            *p = nullptr;
+            failed_ = true;
         }
+        return e;
     }
+    void reset()
+    {
+        for (Chunk &c : chunks_) c.used = 0;
+        failed_ = false;
+    }
+    void trim() { (void)drop_unused(); }
     void release()
     {
-        for (Chunk &c : chunks_) (void)hipFree(c.p);
-        chunks_.clear();
-        total_ = 0;
         reset();
+        (void)drop_unused();
+        separate_ = false;
     }
+    void separate() { separate_ = true; }
+    bool separated() const { return separate_; }
+    bool failed() const { return failed_; }   // an allocation since reset()
     size_t total() const { return total_; }
 
 private:
-    struct Chunk { char *p; size_t size; };
+    struct Chunk { char *p; size_t size, used; };
+    // 1 GiB chunks: 3 % less of a first pass (130 against 134 ms at 512 x 512), but up to 1 GiB left over
+    // for each size of array
+    static constexpr size_t kLarge = 16u << 20, kChunk = 256u << 20;
+
+    static bool cut(Chunk &c, size_t bytes, size_t align, void **p)
+    {
+        const size_t at = (c.used + align - 1) / align * align;
+        if (at + bytes > c.size) return false;
+        *p = c.p + at;
+        c.used = at + bytes;
+        return true;
+    }
+    static hipError_t take(Chunk &c)
+    {
+        const hipError_t e = hipMalloc((void **)&c.p, c.size);
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e;
+    }
+    bool drop_unused()
+    {
+        bool any = false;
+        for (size_t i = chunks_.size(); i-- > 0;) {
+            if (chunks_[i].used) continue;
+            (void)hipFree(chunks_[i].p);
+            total_ -= chunks_[i].size;
+            chunks_.erase(chunks_.begin() + (long)i);
+            any = true;
+        }
+        return any;
+    }
+
     std::vector<Chunk> chunks_;
-    size_t at_ = 0, used_ = 0, total_ = 0;
+    size_t total_ = 0;
+    bool separate_ = false, failed_ = false;
 };
 
 template <typename R>
@@ -432,21 +480,27 @@ struct AdjEngine : AdjEngineBase {
         double *tmp[6] = {};
         int *tf = nullptr;
         const double *src[6] = {x, y, z, u, v, w};
-        for (int i = 0; i < 6; i++) {
-            HIPTRY(dalloc(&tmp[i], n));
-            HIPTRY(hipMemcpyAsync(tmp[i], src[i], n * sizeof(double), kin, c->stream));
-        }
-        HIPTRY(dalloc(&tf, n));
-        HIPTRY(hipMemcpyAsync(tf, flv, n * sizeof(int), kin, c->stream));
-        HIPTRY(hipMemsetAsync(d_err, 0, sizeof(int), c->stream));
-        const double *const raw[6] = {tmp[0], tmp[1], tmp[2], tmp[3], tmp[4], tmp[5]};
-        launch_eng_load<R>(ap, raw, tf, ck[0], n, d_err, c->stream);
-        HIPTRY(hipGetLastError());
         int err = 0;
-        HIPTRY(hipMemcpyAsync(&err, d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        HIPTRY(hipStreamSynchronize(c->stream));
+        auto stage = [&]() -> int {
+            for (int i = 0; i < 6; i++) {
+                HIPTRY(mem.get_beside(&tmp[i], n));
+                HIPTRY(hipMemcpyAsync(tmp[i], src[i], n * sizeof(double), kin, c->stream));
+            }
+            HIPTRY(mem.get_beside(&tf, n));
+            HIPTRY(hipMemcpyAsync(tf, flv, n * sizeof(int), kin, c->stream));
+            HIPTRY(hipMemsetAsync(d_err, 0, sizeof(int), c->stream));
+            const double *const raw[6] = {tmp[0], tmp[1], tmp[2], tmp[3], tmp[4], tmp[5]};
+            launch_eng_load<R>(ap, raw, tf, ck[0], n, d_err, c->stream);
+            HIPTRY(hipGetLastError());
+            HIPTRY(hipMemcpyAsync(&err, d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+            return PICTOR_OK;
+        };
+        const int rc = stage();
+        const hipError_t done = hipStreamSynchronize(c->stream);
         for (int i = 0; i < 6; i++) dfree(tmp[i]);
         dfree(tf);
+        if (rc) return rc;
+        HIPTRY(done);
         if (err) return fail(PICTOR_ERR_ARG, "adjoint: particle outside the physical cells or 2-D z outside [1,2)");
         return PICTOR_OK;
     }
@@ -475,9 +529,9 @@ struct AdjEngine : AdjEngineBase {
         do {
             bool ok = true;
             if (kin == hipMemcpyHostToDevice) {
-                for (int i = 0; i < 7 && ok; i++) ok = dalloc(ds[i], n) == hipSuccess &&
+                for (int i = 0; i < 7 && ok; i++) ok = mem.get_beside(ds[i], n) == hipSuccess &&
                     hipMemcpyAsync(*ds[i], hs[i], n * sizeof(double), kin, s) == hipSuccess;
-                ok = ok && dalloc(&raw.flv, n) == hipSuccess &&
+                ok = ok && mem.get_beside(&raw.flv, n) == hipSuccess &&
                      hipMemcpyAsync(raw.flv, flv, n * sizeof(int), kin, s) == hipSuccess;
             } else {   // the caller's device arrays are read where they are
                 for (int i = 0; i < 7; i++) *ds[i] = const_cast<double *>(hs[i]);
@@ -514,7 +568,8 @@ struct AdjEngine : AdjEngineBase {
                 const long long states = nseg + std::max(seg, 2);
                 const long long need = lay_total * (states * 56 + 2 * 48 + 4LL * seg) + ncell * (48LL * seg + 72);
                 size_t mfree = 0, mtotal = 0;
-                if (lay_total >= 0x7fffffffLL || hipMemGetInfo(&mfree, &mtotal) != hipSuccess || need > 0.95 * ((double)mfree + (double)mem.total())) {
+                if (lay_total >= 0x7fffffffLL || hipMemGetInfo(&mfree, &mtotal) != hipSuccess ||
+                    need > 0.95 * ((double)mfree + (double)mem.total())) {
                     rc = kUseUnsorted;
                     break;
                 }
@@ -842,7 +897,7 @@ struct AdjEngine : AdjEngineBase {
             const bool direct = kout == hipMemcpyDeviceToDevice;
             for (int i = 0; i < 3; i++) {
                 if (direct && h[i]) d[i] = h[i];
-                else HIPTRY(dalloc(&d[i], n));
+                else HIPTRY(mem.get_beside(&d[i], n));
             }
             if (fast) {   // every particle has a slot of checkpoint 0
                 launch_fa_slots<R>(tp, 2, d_base, ck_cnt[0], ck2[0].id, pos, fa[cur], fa[cur], scale, d[0], d[1], d[2], s);
@@ -898,6 +953,15 @@ int adj_forward(pictor_ctx *c, int64_t n, const double *q, const double *x, cons
         if (rc == kUseUnsorted) {
             engine = 1;
             repeats = 0;
+            continue;
+        }
+        if (rc == PICTOR_ERR_HIP && e->mem.failed()) {
+            // no room: once more from nothing, every array on its own
+            if (e->mem.separated()) break;
+            repeats = 0;
+            cf = 1.5;
+            e->release();
+            e->mem.separate();
             continue;
         }
         if (rc != kRetryLayout) break;
