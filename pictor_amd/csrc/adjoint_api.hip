@@ -108,7 +108,13 @@ public:
     void separate() { separate_ = true; }
     bool separated() const { return separate_; }
     bool failed() const { return failed_; }   // an allocation since reset()
-    size_t total() const { return total_; }
+    // bytes of the chunks that nothing has been cut from since reset()
+    size_t unused() const
+    {
+        size_t b = 0;
+        for (const Chunk &c : chunks_) b += c.used ? 0 : c.size;
+        return b;
+    }
 
 private:
     struct Chunk { char *p; size_t size, used; };
@@ -564,12 +570,14 @@ struct AdjEngine : AdjEngineBase {
             for (size_t i = 0; i < ng; i++) counts[i] = cnt[i];
             engine_layout(tp, c->ph.c, counts, cap_factor, h_base, h_cap, lay_total);
             if (!f32) {
-                // the unsorted engine holds n particles a state instead of a layout's slots
+                // the unsorted engine holds n particles a state instead of a layout's slots.  Kept chunks
+                // that setup() cut from are in use, and those that it did not are given back where
+                // they don't suit
                 const long long states = nseg + std::max(seg, 2);
-                const long long need = lay_total * (states * 56 + 2 * 48 + 4LL * seg) + ncell * (48LL * seg + 72);
+                const long long need = lay_total * (states * 56 + 2 * 48 + 4LL * seg) + ncell * (48LL * seg + 72) + 4 * n;
                 size_t mfree = 0, mtotal = 0;
                 if (lay_total >= 0x7fffffffLL || hipMemGetInfo(&mfree, &mtotal) != hipSuccess ||
-                    need > 0.95 * ((double)mfree + (double)mem.total())) {
+                    need > 0.95 * ((double)mfree + (double)mem.unused())) {
                     rc = kUseUnsorted;
                     break;
                 }
@@ -956,8 +964,11 @@ int adj_forward(pictor_ctx *c, int64_t n, const double *q, const double *x, cons
             continue;
         }
         if (rc == PICTOR_ERR_HIP && e->mem.failed()) {
-            // no room: once more from nothing, every array on its own
-            if (e->mem.separated()) break;
+            // no room: once more from nothing, every array on its own; then FP64 with the engine
+            // whose states are smaller
+            const bool again = e->mem.separated();
+            if (again && !(std::is_same<R, double>::value && engine == 0)) break;
+            if (again) engine = 1;
             repeats = 0;
             cf = 1.5;
             e->release();

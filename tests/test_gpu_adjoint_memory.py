@@ -187,3 +187,24 @@ def test_kept_memory_makes_room(card):
         assert Lb == pytest.approx(La, rel=1e-12)
         for a, b in zip(*card.part_out):
             assert float((a - b).norm()) <= 1e-11 * float(b.norm())
+
+
+def test_fields_count_as_used(card):
+    # a large grid with few particles: the field checkpoints that the pass already holds are no room for
+    # its bins, and the unsorted engine runs where those do not fit
+    n, count = (2048, 2048), 100000
+    P = {k: v[:: COUNT // count][:count].contiguous() for k, v in card.P.items()}
+    out = [[torch.empty_like(P["x"]) for _ in range(3)] for _ in range(2)]
+    with Simulation(*n, epc=8, form="fp64", tile=16) as sim:
+        L, stats = _device_pass(sim, P, out[0], 8, 1)
+        assert stats["engine"] == 0.0
+    with Simulation(*n, epc=8, form="fp64", tile=16) as sim:
+        hold = card.leave(0.96 * stats["device_bytes"])
+        Lb, least = _device_pass(sim, P, out[1], 8, 1)
+        say("sorted %.2f GiB, unsorted %.2f" % (stats["device_bytes"] / 2**30, least["device_bytes"] / 2**30))
+        assert least["engine"] == 1.0
+        del hold
+        torch.cuda.empty_cache()
+    assert Lb == pytest.approx(L, rel=1e-12)
+    for a, b in zip(*out):
+        assert float((a - b).norm()) <= 1e-11 * float(b.norm())
