@@ -481,18 +481,24 @@ int do_e_phase(pictor_ctx *c, bool curl, bool add, bool halo = true)
     return PICTOR_OK;
 }
 
-// the second buffers of the fused step
-int ensure_field_pairs(pictor_ctx *c)
+// the second buffers of the fused step; false: no room for them
+bool ensure_field_pairs(pictor_ctx *c)
 {
-    if (c->J2[2]) return PICTOR_OK;
+    if (c->J2[2]) return true;
     const size_t n = (size_t)c->g.ncell, rs = c->form == PICTOR_FORM_FP64 ? sizeof(double) : sizeof(float);
+    bool ok = true;
+    for (int i = 0; i < 3 && ok; i++)
+        ok = hipMalloc(&c->E2[i], n * rs) == hipSuccess && hipMalloc(&c->B2[i], n * rs) == hipSuccess &&
+             (c->form == PICTOR_FORM_FP64 || dalloc(&c->Elo2[i], n) == hipSuccess) &&
+             hipMalloc(&c->J2[i], n * sizeof(double)) == hipSuccess;
+    if (ok) return true;
+    (void)hipGetLastError();
     for (int i = 0; i < 3; i++) {
-        if (!c->E2[i]) HIPTRY(hipMalloc(&c->E2[i], n * rs));
-        if (!c->B2[i]) HIPTRY(hipMalloc(&c->B2[i], n * rs));
-        if (c->form != PICTOR_FORM_FP64 && !c->Elo2[i]) HIPTRY(dalloc(&c->Elo2[i], n));
-        if (!c->J2[i]) HIPTRY(hipMalloc(&c->J2[i], n * sizeof(double)));
+        dfree(c->E2[i]); dfree(c->B2[i]); dfree(c->Elo2[i]); dfree(c->J2[i]);
+        c->E2[i] = c->B2[i] = c->J2[i] = nullptr;
+        c->Elo2[i] = nullptr;
     }
-    return PICTOR_OK;
+    return false;
 }
 
 void swap_fields(pictor_ctx *c, bool current)
@@ -519,8 +525,8 @@ FieldStepP<R> field_args(pictor_ctx *c, bool in_place)
 }
 
 // Whole steps of a periodic box: per step the push and one launch for the fields (three in
-// place for the 3-D Lehe update), with the second half step of B, E and the next step's first
-// half step in it.  Up to kRun steps are enqueued before the host waits: a step that spills or
+// place for the 3-D Lehe update, and where the card has no room for second buffers), with the second
+// half step of B, E and the next step's first half step in it.  Up to kRun steps are enqueued before the host waits: a step that spills or
 // fails closes the gate of the ones behind it, which then do nothing, and the host carries on
 // from there after the re-layout.  The last step of a call leaves J folded, as the phases do,
 // and B at the step's end.  At 32 x 32 (FP64, 4 particles per cell) a step took 75 us with a
@@ -529,11 +535,10 @@ template <typename R>
 int step_periodic(pictor_ctx *c, int nsteps)
 {
     constexpr int kRun = 32;
-    const bool in_place = c->g.ndim == 3 && c->ph.fdtd != PICTOR_FDTD_YEE;
+    const bool in_place = (c->g.ndim == 3 && c->ph.fdtd != PICTOR_FDTD_YEE) || !ensure_field_pairs(c);
     const bool filter = c->curr_filter > 0;
     hipStream_t s = c->stream;
-    int rc = in_place ? PICTOR_OK : ensure_field_pairs(c);
-    if (rc) return rc;
+    int rc;
     while (c->sev.size() < 2 * kRun + 2) {
         hipEvent_t e;
         HIPTRY(hipEventCreate(&e));

@@ -77,3 +77,44 @@ def test_overflow_inside_a_run(form, ndim, n, fdtd):
             assert np.array_equal(a[k], b[k]) and np.array_equal(a[k], c[k]), k
         else:
             assert np.abs(a[k] - b[k]).max() <= 1e-9 * np.abs(b[k]).max(), k
+
+
+def test_step_without_room_for_second_buffers():
+    # a card too full for the second field buffers: the step runs in place, with the same bits
+    import torch
+
+    cases = [((1024, 1024, 1), 2, dict()), ((1024, 768, 1), 2, dict(fdtd="lehe", curr_filter=1)), ((96, 96, 96), 3, dict())]
+
+    def start(n, ndim, more):
+        sim = Simulation(*n, ndim=ndim, epc=2, form="fp32_split", **more)
+        sim.upload_particles(**setup_weibel(*n, ndim=ndim, epc=2, drift=0.5, uth=0.2, seed=8))
+        return sim
+
+    want = []
+    for c in cases:
+        with start(*c) as sim:
+            lean = sim.memory_bytes()
+            sim.step(5)
+            want.append(sim.download_fields())
+            assert sim.memory_bytes() > lean
+    sims = [start(*c) for c in cases]
+    torch.cuda.empty_cache()
+    torch.cuda.synchronize()
+    held = [torch.empty(torch.cuda.mem_get_info()[0] - (64 << 20), dtype=torch.uint8, device="cuda")]
+    try:
+        while True:     # more than the runtime says is there
+            held.append(torch.empty(22 << 20, dtype=torch.uint8, device="cuda"))
+    except torch.OutOfMemoryError:
+        held.pop()
+        torch.cuda.empty_cache()
+    lean = [sim.memory_bytes() for sim in sims]
+    for sim in sims:
+        sim.step(5)
+    assert [sim.memory_bytes() for sim in sims] == lean
+    del held
+    torch.cuda.empty_cache()
+    for sim, F in zip(sims, want):
+        G = sim.download_fields()
+        sim.close()
+        for k in F:
+            assert np.array_equal(G[k], F[k]), k
