@@ -1464,6 +1464,8 @@ int pictor_memory_bytes(pictor_ctx *c, int64_t *bytes)
         // FP64 E, B, J; the particle slots (FP64 record 60 B, split record 32 B)
         const long long per = (c->form == PICTOR_FORM_FP64) ? 60 : 32;
         *bytes = c->g.ncell * 9 * 8 + c->cm.cap * per;
+        for (int i = 0; i < 3; i++)   // the open run's second E and B
+            *bytes += ((c->E2[i] ? 1 : 0) + (c->B2[i] ? 1 : 0)) * c->g.ncell * 8;
         return PICTOR_OK;
     }
     const long long rs = (c->form == PICTOR_FORM_FP64) ? 8 : 4;

@@ -718,3 +718,14 @@ def test_error_inside_an_open_run_stops_behind_that_push(form):
         assert np.array_equal(fa[k], fb[k]), k
     for k in pa:
         assert np.array_equal(pa[k], pb[k]), k
+
+
+@pytest.mark.parametrize("form", ["fp32_split", "fp64"])
+def test_memory_report_counts_the_window_run(form):
+    # the moving window's run keeps a second set of E and B: six FP64 arrays
+    say(f"[case] cylm memory report {form}")
+    with Simulation(18, 2, 32, ndim=3, epc=4, c=0.4, c_ompe=10.0, form=form, geometry="cyl_modal") as sim:
+        sim.moving_window(True)
+        before = sim.memory_bytes()
+        sim.step(3)
+        assert sim.memory_bytes() == before + 6 * 8 * int(np.prod(sim.shape))
