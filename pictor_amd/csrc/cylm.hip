@@ -2058,10 +2058,18 @@ int cylm_step(pictor_ctx *c, int nsteps)
     int rc = cylm_setup(c);
     // the open-ended run: a second set of E and B to shift into, and at most one shift a step
     bool open = c->cq.zopen && st.win_on && c->ph.c < 1.0;
-    for (int i = 0; i < 3 && open; i++)
-        open = (c->E2[i] || dalloc((double **)&c->E2[i], c->g.ncell) == hipSuccess) &&
-               (c->B2[i] || dalloc((double **)&c->B2[i], c->g.ncell) == hipSuccess);
-    if (c->cq.zopen && !open) (void)hipGetLastError();
+    if (open && !c->B2[2]) {
+        for (int i = 0; i < 3 && open; i++)
+            open = dalloc((double **)&c->E2[i], c->g.ncell) == hipSuccess &&
+                   dalloc((double **)&c->B2[i], c->g.ncell) == hipSuccess;
+        if (!open) {   // no room: back with what there was, a step at a time
+            (void)hipGetLastError();
+            for (int i = 0; i < 3; i++) {
+                dfree(c->E2[i]); dfree(c->B2[i]);
+                c->E2[i] = c->B2[i] = nullptr;
+            }
+        }
+    }
     for (int done = 0; done < nsteps && !rc;) {
         const bool one = (double)(st.win_steps + 1) * c->ph.c < (double)(st.win_shift + 2);
         if (open && one) {

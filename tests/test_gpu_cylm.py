@@ -729,3 +729,45 @@ def test_memory_report_counts_the_window_run(form):
         before = sim.memory_bytes()
         sim.step(3)
         assert sim.memory_bytes() == before + 6 * 8 * int(np.prod(sim.shape))
+
+
+def test_window_run_without_room_for_second_fields():
+    # a card with room for some of the second E and B: none of them stays, the steps run one at a time
+    # with the same bits, and the run takes them when there is room again
+    import torch
+
+    say("[case] cylm window run on a full card")
+
+    def make():
+        sim = Simulation(500, 2, 4000, ndim=3, epc=4, c=0.4, c_ompe=10.0, form="fp32_split", geometry="cyl_modal", dr=2.0)
+        sim.cyl_plasma(100, 3, 200, 4, seed=3)
+        sim.moving_window(True)
+        sim.cyl_laser(0.5, 8.0, 2.0, 3.0, 150.0)
+        sim.ResetCurrent()
+        sim.MoveDepositPrtl()      # allocates the push's node copy
+        sim.ExchangePrtl()
+        return sim
+
+    with make() as sim:
+        lean, array = sim.memory_bytes(), 8 * int(np.prod(sim.shape))
+        sim.step(7)
+        want, full = sim.download_fields(), sim.memory_bytes()
+    assert full == lean + 6 * array
+    with make() as sim:
+        torch.cuda.empty_cache()
+        held = [torch.empty(torch.cuda.mem_get_info()[0] - (256 << 20), dtype=torch.uint8, device="cuda")]
+        try:
+            while True:     # more than the runtime says is there
+                held.append(torch.empty(22 << 20, dtype=torch.uint8, device="cuda"))
+        except torch.OutOfMemoryError:
+            del held[-(3 * array // (22 << 20)):]
+            torch.cuda.empty_cache()
+        sim.step(7)
+        assert sim.memory_bytes() == lean
+        del held
+        torch.cuda.empty_cache()
+        got = sim.download_fields()
+        sim.step(1)
+        assert sim.memory_bytes() == full
+    for k in want:
+        assert np.array_equal(got[k], want[k]), k
