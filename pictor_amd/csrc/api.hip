@@ -611,7 +611,8 @@ int step_periodic(pictor_ctx *c, int nsteps)
 
 int choose_tile(const pictor_config *cfg)
 {
-    // 2-D: tile 16 (512-lane workgroups, 35 KB of LDS: four per CU) is the fastest push
+    // 2-D: tile 16 (512-lane workgroups; by their registers three per CU in the split form, 74 to
+    // 78 of them, and two in FP64, 98) is the fastest push
     // in both forms once the grid has 1024 tiles of it; smaller grids take tile 8 for
     // more workgroups.  3-D windows are (T+3)^3 / (T+5)^3 nodes: 8 is the largest tile
     // whose LDS fits

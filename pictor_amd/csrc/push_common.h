@@ -8,12 +8,6 @@ namespace pushdev {
 __device__ inline double dmin(double a, double b) { return (b < a) ? b : a; }
 __device__ inline double dmax(double a, double b) { return (b > a) ? b : a; }
 
-__device__ inline unsigned long long lanemask_lt()
-{
-    unsigned lane = __lane_id();
-    return (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-}
-
 // an error of this step, and a spilled particle: both stop the steps enqueued behind it
 __device__ inline void flag_error(const SpillP &sp, int bits)
 {

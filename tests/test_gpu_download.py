@@ -1,5 +1,5 @@
 """Downloads through the pinned ring: results on both sides of the size from which host threads
-copy (2 MiB), arrays of less and more than one 1 MiB piece, more pieces than the ring holds,
+copy (6 MiB: 288 x 288 and 288 x 296), arrays of less and more than one 1 MiB piece, more pieces than the ring holds,
 arrays left out, and several contexts from several threads."""
 import ctypes
 import threading
@@ -33,7 +33,7 @@ def _expect(form, name, f):
 
 
 @pytest.mark.parametrize("form", ["fp32_split", "fp64"])
-@pytest.mark.parametrize("n", [(8, 8), (160, 160), (168, 160), (368, 360), (1024, 704)])
+@pytest.mark.parametrize("n", [(8, 8), (160, 160), (168, 160), (288, 288), (288, 296), (368, 360), (1024, 704)])
 def test_fields(form, n):
     say(form, n)
     with Simulation(*n, form=form) as sim:
