@@ -59,7 +59,8 @@ template <> struct FaState<double> { using T = PartE64; };
 // FP64 forward push of the tile-sorted engine (adjoint_fast.hip), tile 8 or 16: the particles
 // of every bin of A into the bins of O, dst[input slot] = output slot (dst may be null; -1 for a
 // particle that found its bin full, which is counted in sp.count and dropped: the caller
-// repeats the pass with larger bins), the current into J.
+// repeats the pass with larger bins, or, with kErrCapacity in sp.err, goes on without bins),
+// the current into J.
 void launch_fa_push64(const GridP &g, const TileP &tp, const AdjP &ap, double *const E[3], double *const B[3],
                       double *const J[3], PartE64 A, PartE64 O, BinsP bins, SpillP sp, int *dst, hipStream_t s);
 // the caller's particles into the centre bins of an FP64 state (tile_of from launch_raw_tiles_f64;

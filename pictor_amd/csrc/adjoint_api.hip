@@ -315,6 +315,7 @@ struct AdjEngine : AdjEngineBase {
     PartSplit spill{};
     int spill_cap = 0;
     int *d_spill = nullptr;
+    int *d_stop = nullptr;              // the first step of the forward pass that overflowed (Gate)
 
     Arena mem;
 
@@ -349,7 +350,7 @@ struct AdjEngine : AdjEngineBase {
         sfE.clear(); sfB.clear();
         fa[0] = fa[1] = EPart<R>{};
         spill = PartSplit{};
-        d_base = nullptr; d_cap = nullptr; pos = nullptr; d_spill = nullptr;
+        d_base = nullptr; d_cap = nullptr; pos = nullptr; d_spill = d_stop = nullptr;
         h_base.clear(); h_cap.clear();
         lay_total = 0;
         partial = nullptr;
@@ -467,6 +468,7 @@ struct AdjEngine : AdjEngineBase {
             HIPTRY(alloc_state(mem, spill, spill_cap, false, true, bytes));
         }
         HIPTRY(mem.get(&d_spill, 1));
+        HIPTRY(mem.get(&d_stop, 1));
         bytes += (long long)(nseg + ns) * 4 * nb + 12LL * nb + (long long)seg * 4 * lay_total +
                  (long long)seg * 6 * sizeof(R) * ncell + 4 * n;
         return PICTOR_OK;
@@ -622,11 +624,12 @@ struct AdjEngine : AdjEngineBase {
     }
 
     // the push of one step of the tile-sorted engine: state (in, cin) -> (out, cout) in the
-    // fields fE, fB; dst (may be null) records the slots
-    void push_bins(R *const *fE, R *const *fB, State in, const int *cin, State out, int *cout, int *dst)
+    // fields fE, fB; dst (may be null) records the slots.  Step t >= 0 of the forward pass: an
+    // overflow ends the pass, and what is enqueued behind that step does nothing
+    void push_bins(R *const *fE, R *const *fB, State in, const int *cin, State out, int *cout, int *dst, int t)
     {
         BinsP bins{d_base, d_cap, cin, cout};
-        SpillP sp{d_spill, spill_cap, d_err};
+        SpillP sp{d_spill, spill_cap, d_err, t >= 0 ? d_stop : nullptr, t};
         if constexpr (std::is_same<R, float>::value)
             launch_push2d_split_track(c->tp.T, c->g, c->ph, c->tp, fE, fB, J, in, out, bins, spill, sp, dst, c->stream);
         else
@@ -645,14 +648,16 @@ struct AdjEngine : AdjEngineBase {
 
     // the rest of a step's fields from (fE, fB, Elo, J) into (nE, nB, Elo2), and with `next` the
     // first half step of the following one; Elo and J swap with their second buffers, J cleared
-    void finish_fields(R *const *fE, R *const *fB, R *const *nE, R *const *nB, bool next)
+    void finish_fields(R *const *fE, R *const *fB, R *const *nE, R *const *nB, bool next, int t)
     {
         hipStream_t s = c->stream;
+        const Gate gate{t >= 0 ? d_stop : nullptr, t};
         if (c->curr_filter > 0) {
-            launch_current_fold<double>(c->g, J, s);
-            launch_smoothen_current(c->g, c->curr_filter, J, Jt, s);
+            launch_current_fold<double>(c->g, J, s, gate);
+            launch_smoothen_current(c->g, c->curr_filter, J, Jt, s, gate);
         }
         FieldStepP<R> P{};
+        P.gate = gate;
         for (int i = 0; i < 3; i++) {
             P.E[i] = fE[i]; P.B[i] = fB[i]; P.L[i] = Elo[i]; P.J[i] = J[i];
             P.En[i] = nE[i]; P.Bn[i] = nB[i]; P.Ln[i] = Elo2[i]; P.Jz[i] = J2[i];
@@ -677,6 +682,8 @@ struct AdjEngine : AdjEngineBase {
         if (h[1] & kErrPrecision)
             return fail(PICTOR_ERR_CAPACITY, "adjoint: current at a node exceeded the exact fixed-point range");
         if (h[0] > 0 || (h[1] & kErrCapacity)) {
+            // FP64: a bin that larger centre bins would not help (k_fa_push64)
+            if (forward_pass && std::is_same<R, double>::value && (h[1] & kErrCapacity)) return kUseUnsorted;
             if (forward_pass) return kRetryLayout;
             return fail(PICTOR_ERR_CAPACITY, "adjoint: tile bins overflowed while recomputing a segment");
         }
@@ -687,6 +694,7 @@ struct AdjEngine : AdjEngineBase {
     {
         HIPTRY(hipMemsetAsync(d_err, 0, sizeof(int), c->stream));
         if (d_spill) HIPTRY(hipMemsetAsync(d_spill, 0, sizeof(int), c->stream));
+        if (d_stop) HIPTRY(hipMemsetAsync(d_stop, 0x7f, sizeof(int), c->stream));
         return PICTOR_OK;
     }
 
@@ -786,8 +794,8 @@ struct AdjEngine : AdjEngineBase {
                 const bool ends = (t + 1) % seg == 0, to_ck = ends && k1 < nseg;
                 State b = to_ck ? ck2[k1] : st2[1 + (t % 2)];
                 int *bc = to_ck ? ck_cnt[k1] : cntv[1 + (t % 2)];
-                push_bins(E, B, a, ac, b, bc, nullptr);
-                finish_fields(E, B, E2, B2, !ends && t + 1 < nsteps);
+                push_bins(E, B, a, ac, b, bc, nullptr, t);
+                finish_fields(E, B, E2, B2, !ends && t + 1 < nsteps, t);
                 for (int i = 0; i < 3; i++) {
                     std::swap(E[i], E2[i]);
                     std::swap(B[i], B2[i]);
@@ -859,10 +867,10 @@ struct AdjEngine : AdjEngineBase {
                 auto S = [&](int j) { return j == 0 ? ck2[k] : st2[j]; };
                 auto C = [&](int j) { return j == 0 ? ck_cnt[k] : cntv[j]; };
                 for (int j = 0; j < L; j++) {
-                    push_bins(&sfE[3 * j], &sfB[3 * j], S(j), C(j), st2[j + 1], cntv[j + 1], dstv[j]);
+                    push_bins(&sfE[3 * j], &sfB[3 * j], S(j), C(j), st2[j + 1], cntv[j + 1], dstv[j], -1);
                     // the fields after the segment's last push are in the next checkpoint
                     if (j + 1 < L)
-                        finish_fields(&sfE[3 * j], &sfB[3 * j], &sfE[3 * (j + 1)], &sfB[3 * (j + 1)], true);
+                        finish_fields(&sfE[3 * j], &sfB[3 * j], &sfE[3 * (j + 1)], &sfB[3 * (j + 1)], true, -1);
                 }
                 HIPTRY(hipGetLastError());
                 HIPTRY(hipEventRecord(ev[1], s));

@@ -108,6 +108,7 @@ __global__ __launch_bounds__(BS) void k_fa_push64(GridP g, TileP tp, AdjP ap, co
     __shared__ double sJ[3][WW];
     __shared__ int sStart[10], sCnt[9], sDstCap[9], sDstBin[9];
     __shared__ unsigned sSrc[9], sDstBase[9];
+    if (sp.stop && *sp.stop < sp.step) return;
     const int tile = tile_remap(tp, blockIdx.x);
     const int tx = tile % tp.ntx, ty = tile / tp.ntx;
     const int iw = 1 + tx * T, jw = 1 + ty * T, cx0 = tx * T - 2, cy0 = ty * T - 2;
@@ -201,7 +202,10 @@ __global__ __launch_bounds__(BS) void k_fa_push64(GridP g, TileP tp, AdjP ap, co
                 O.p.u[o] = un[0]; O.p.v[o] = un[1]; O.p.w[o] = un[2];
                 to = (int)o;
             } else if (d >= 0) {
-                atomicAdd(sp.count, 1);
+                // centre bins grow with the tile's own population when the pass is repeated; a side
+                // bin, or the centre of a nearly empty tile, would only overflow again
+                spill_slot(sp);
+                if (d != 4 || sDstCap[4] <= 80) atomicOr(sp.err, (int)kErrCapacity);
             }
             if (dst) dst[slot_in] = to;
         }

@@ -69,6 +69,19 @@ def test_bins_that_never_fit():
     _same("fp32_split", b, _fresh("fp32_split", n, "sorted", Q, 6, 3))
 
 
+def test_bins_that_grow_too_little():
+    # a dense tile flows into one with a dozen particles: its centre overflows at 12 times that count too
+    n = (32, 16)
+    dense, thin = setup_weibel(*n, epc=10, drift=0.0, uth=0.05, seed=4), setup_weibel(*n, epc=2, drift=0.0, uth=0.05, seed=5)
+    tile = (dense["x"] >= 11.0) & (dense["x"] < 19.0) & (dense["y"] < 11.0)
+    some = np.random.default_rng(3).random(len(thin["x"])) < 0.06
+    P = {k: np.concatenate([dense[k][tile], thin[k][some]]) for k in dense}
+    P["u"] += 0.3
+    a = _fresh("fp64", n, "sorted", P, 30, 7)
+    assert a[2]["engine"] == 1.0
+    _same("fp64", a, _fresh("fp64", n, "unsorted", P, 30, 7))
+
+
 @pytest.mark.parametrize("form", ["fp64", "fp32_split"])
 def test_passes_of_one_context(form):
     n = (48, 40)
