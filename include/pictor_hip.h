@@ -289,8 +289,8 @@ int pictor_adjoint_stats(pictor_ctx *ctx, double out[10]);
 /* Engine: 0 = tile-sorted (default; the particles in tile bins, the field and
  * the current of a tile in LDS, the reverse step over the same bins; FP32 split
  * form: every forward step the production push, tile edge 8, 16 or 32; FP64:
- * tile edge 8 or 16 and memory for the bins of every kept state, otherwise the
- * unsorted engine), 1 = unsorted (one thread per particle, global atomics).
+ * tile edge 8 or 16, memory for the bins of every kept state and bins that hold
+ * the flow from tile to tile, otherwise the unsorted engine), 1 = unsorted (one thread per particle, global atomics).
  * Takes effect at the next pictor_adjoint_forward. */
 int pictor_adjoint_engine(pictor_ctx *ctx, int32_t engine);
 int pictor_adjoint_release(pictor_ctx *ctx);
